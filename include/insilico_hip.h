@@ -369,8 +369,8 @@ int ins_cell_eval(ins_ctx* ctx, int quantity, const double* xi, const double* u,
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory: code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc.  The FP64 Jacobi-PCG of ins_solve(INS_SOLVE_FP64,
- * INS_FMT_CSR) -- same kernels, grids and reduction order, so the same
- * iterates -- on a CSR system held in caller-owned DEVICE arrays of GPU
+ * INS_FMT_CSR) -- the same row products, row segments and order of all sums,
+ * so the same iterates -- on a CSR system held in caller-owned DEVICE arrays of GPU
  * `device`: row_ptr (n+1, row_ptr[n] = nnz), col_idx (nnz, ascending per
  * row), val (nnz), b (n) are read, x (n) receives the solution; stream is a
  * hipStream_t (NULL = the default stream) and the call returns after the

@@ -81,6 +81,8 @@ static void release_all(Ctx* c)
     release(c, c->sell.vs64); release(c, c->sell.spw); release(c, c->sell.anode);
     release(c, c->sell.vs); release(c, c->sell.su); release(c, c->sell.smap);
     release(c, c->emask);
+    release(c, c->res.words); release(c, c->res.wlen); release(c, c->res.woff);
+    release(c, c->res.own0); release(c, c->res.wlist); release(c, c->res.lcol);
 }
 
 // A context detached from a server may still be named by the batched work
@@ -96,6 +98,7 @@ int wait_server_release(Ctx* c)
 
 static void invalidate_pattern(Ctx* c)
 {
+    c->pattern_gen++;
     c->have_pattern = false;
     c->have_matrix = false;
     c->have_rhs = false;

@@ -68,8 +68,13 @@ struct Scal {
     int stop;        // FP64: converged in K3 of the last iteration; the next
                      // K1 turns it into done (K3 itself never reads it, so
                      // every block of that K3 still does its x update)
-    int pad_;
+    int abort;       // resident: a block waited in vain for the others, the
+                     // solve is to be repeated by the segment kernels
 };
+
+// rep_at of a resident solve: the replacement comes next, whatever the
+// iteration (also the iteration index its kernels are launched with)
+constexpr int RES_REPLACE = INT32_MAX - 1;
 
 // SELL-64 matrix: 64-row slices, values column-major inside a slice; every
 // slice uses one column-offset list (col = row + delta) from a dictionary.
@@ -135,6 +140,19 @@ struct Sell {
     DArr<int32_t> anode;
 };
 
+// Segments and windows of the resident solves (resident.hpp)
+struct Resident {
+    DArr<uint64_t> words;    // device-wide sums
+    uint32_t epoch = 0;      // of the next sum
+    // windows of the CSR pattern csr_gen
+    uint64_t csr_gen = 0;
+    int csr_seg_B = 0, csr_seg_R = 0;
+    bool csr_ok = false;
+    int csr_wmax = 0, csr_maxlen = 0;
+    DArr<int32_t> wlen, woff, own0, wlist;
+    DArr<uint16_t> lcol;     // place of every CSR entry's column in its window
+};
+
 struct Ctx {
     int device = 0;
     int n_cu = 256;         // compute units of the device
@@ -182,6 +200,7 @@ struct Ctx {
     bool dofs_match() const { return have_dofs && n_active == dof_n_active; }
 
     // pattern
+    uint64_t pattern_gen = 1;  // changes whenever row_ptr / col do
     bool have_pattern = false;
     // the CSR came from ins_set_csr (values of unknown symmetry) rather than
     // from the element assembly (symmetric pattern and values)
@@ -269,6 +288,7 @@ struct Ctx {
     bool fe_slab = false;    // ... in 64-element slabs (heat::Laplace Q1) or element-major
     DArr<double> stage_ff;   // face force vectors
     Sell sell;
+    Resident res;
 
     // solver state
     DArr<double> x, r, p, q, t64;

@@ -30,7 +30,7 @@
 #include <hip/hip_ext.h>
 #include <rocsolver/rocsolver.h>
 
-#include "common.hpp"
+#include "resident.hpp"
 
 // Multiply-adds fuse only within one source expression (s += a * b is one
 // FMA everywhere).  With contraction left to the backend, whether a product
@@ -43,102 +43,14 @@ namespace ins {
 
 namespace {
 
-constexpr int VB = 512;       // threads per block of the vector kernels
-constexpr int SB = 256;       // threads per block of the SpMV kernels
-constexpr int MAXG = 2048;    // max blocks of a partial-producing kernel
 constexpr int CHUNK = 32;     // FP64 iterations between host checks
 constexpr int MCHUNK = 16;    // mixed: iterations between host checks
-// partial slots
-constexpr int P_PQ = 0, P_RR = 1, P_RZ = 2, P_TT = 3, P_BB = 4, NSLOT = 5;
-
-__device__ inline double wave_sum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-// sum of v over the block, returned to every thread (fixed order)
-template <int NV>
-__device__ inline void block_allsum(double (&v)[NV])
-{
-    __shared__ double sh[NV][16];
-#pragma unroll
-    for (int k = 0; k < NV; k++) v[k] = wave_sum(v[k]);
-    const int nw = blockDim.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int k = 0; k < NV; k++) sh[k][threadIdx.x >> 6] = v[k];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NV; k++) {
-        double s = 0.;
-        for (int w = 0; w < nw; w++) s += sh[k][w];
-        v[k] = s;
-    }
-}
-
-// A block's place in the decomposition of one solve: its index and the
-// number of blocks.  A plain launch uses blockIdx/gridDim; a batched launch
-// (several solves in one grid) gives every solve the decomposition it has
-// alone, so its sums, and hence its iterates, do not depend on the batch.
-struct Blk {
-    int id, n;
-};
-__device__ inline Blk grid_blk() { return Blk{(int)blockIdx.x, (int)gridDim.x}; }
-
-// one partial per block
-template <int NV>
-__device__ inline void block_partials(double (&v)[NV], double* part, const int (&slot)[NV],
-                                      Blk b = grid_blk())
-{
-    block_allsum<NV>(v);
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int k = 0; k < NV; k++) part[slot[k] * MAXG + b.id] = v[k];
-}
-
-// every block: the same total of cnt partials of the given slots
-template <int NV>
-__device__ inline void totals(const double* part, int cnt, const int (&slot)[NV], double (&t)[NV])
-{
-#pragma unroll
-    for (int k = 0; k < NV; k++) t[k] = 0.;
-    for (int i = threadIdx.x; i < cnt; i += blockDim.x)
-#pragma unroll
-        for (int k = 0; k < NV; k++) t[k] += part[slot[k] * MAXG + i];
-    block_allsum<NV>(t);
-}
-
-__device__ inline bool leader(Blk b = grid_blk()) { return b.id == 0 && threadIdx.x == 0; }
-
-// this thread's share of totals<NV> (the loads only; block_allsum finishes
-// it), so that a kernel can issue them together with its other loads
-template <int NV>
-__device__ inline void totals_share(const double* part, int cnt, const int (&slot)[NV],
-                                    double (&t)[NV])
-{
-#pragma unroll
-    for (int k = 0; k < NV; k++) t[k] = 0.;
-    for (int i = threadIdx.x; i < cnt; i += blockDim.x)
-#pragma unroll
-        for (int k = 0; k < NV; k++) t[k] += part[slot[k] * MAXG + i];
-}
-
-// index of the calling wavefront within its block, as a wave-uniform value:
-// slice indices derived from it stay in scalar registers, so the per-slice
-// offset, pattern and column-offset reads go through the scalar cache rather
-// than through one vector load per lane
-__device__ inline int wave_in_block() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
 // Workgroups are placed on the 8 XCDs round-robin by block id.  Each XCD
 // owns one contiguous eighth of the items (rows or slices) and its blocks
 // sweep that eighth together in grid-stride order: 8 sequential streams,
 // one per XCD, with the x gathers of the SpMV and the vectors reused by the
 // next kernel local to that XCD's L2.
-constexpr int NXCD = 8;
-
 struct Sweep {
     int64_t first;   // first item of this block
     int64_t end;     // end of the XCD's range
@@ -196,23 +108,6 @@ struct SellView {
 // position = slice_base + (k/4)*256 + lane*4 + k%4, so a lane reads 4 entries
 // of its row with one 16-byte load (32 bytes for FP64) and a wavefront reads
 // 1 KB contiguous.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x2 __attribute__((ext_vector_type(2)));
-
-template <typename TV>
-__device__ inline void load4(const TV* p, TV (&o)[4])
-{
-    if constexpr (sizeof(TV) == 4) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(p);
-        o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
-    } else {
-        const f64x2 a = *reinterpret_cast<const f64x2*>(p);
-        const f64x2 b = *reinterpret_cast<const f64x2*>(p + 2);
-        o[0] = a.x; o[1] = a.y; o[2] = b.x; o[3] = b.y;
-    }
-}
-
-
 // one lane per row of a 64-row slice; all rows of a slice share one
 // column-offset list (the union of their own lists, values zero-padded), so
 // the offsets are wave-uniform and read with scalar loads.  Padded entries
@@ -521,9 +416,7 @@ __device__ inline TA csr_row(int64_t row, int sub, const int32_t* __restrict__ r
 #pragma unroll
         for (int j = 0; j < 4; j++) s += (TA)vv[j] * (TA)xx[j];
     }
-#pragma unroll
-    for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, LPR);
-    return s;
+    return group_sum<LPR>(s);
 }
 
 // Symmetric node-block slices (vector problems, one lane per node of a
@@ -1031,11 +924,14 @@ struct V16<double> {
 
 // K2: alpha from the p.q partials; r -= alpha q; r.r, r.z partials (the
 // x update waits for K3)
-template <typename TX, typename TD>
+// SD > 0: on the segments of resident.hpp instead (b.id: the segment, sl: its
+// slices, SD components of n items), the items and sums of the resident
+// kernel
+template <typename TX, typename TD, int SD = 0>
 __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* __restrict__ r,
                                       const TX* __restrict__ p, const TX* __restrict__ q,
                                       const TD* __restrict__ dinv, double* part, int g_pq,
-                                      Scal* sc, int it)
+                                      Scal* sc, int it, int sl_seg = 0)
 {
     // everything this kernel waits on before its sweep -- the scalars of
     // the last iterations and this thread's share of K1's p.q partials --
@@ -1068,15 +964,17 @@ __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* 
                 // true residual; once the FP32 recursion has converged or
                 // drifted, restart from p = D^-1 r
                 sc->restart = (sc->conv32 || t[0] > g_restart_ratio * sc->rr) ? 1 : 0;
-                sc->rho[(it + 1) & 1] = t[1];
+                sc->rho[0] = t[1];
+                sc->rho[1] = t[1];
                 sc->rr = t[0];
                 sc->rref = t[0];
             }
             sc->conv32 = 0;
+            if (it == RES_REPLACE) sc->rep_at = INT_MAX;
         }
         return;
     }
-    if (done) return;
+    if (done || it == RES_REPLACE) return;
     if (stop) {
         // converged in the last K3: done from here on
         if (leader(b)) sc->done = 1;
@@ -1103,6 +1001,19 @@ __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* 
     constexpr int W = V16<TX>::W;
     const TX alpha = (TX)ad;
     double rr = 0., rz = 0.;
+    if constexpr (SD > 0) {
+        seg_items<SD>(b.id, sl_seg, n, [&](int64_t i) {
+            const TX ri = r[i] - alpha * q[i];
+            r[i] = ri;
+            const TX zi = dinv[i] * ri;
+            rr += (double)ri * (double)ri;
+            rz += (double)ri * (double)zi;
+        });
+        double v[2] = {rr, rz};
+        const int sl[2] = {P_RR, P_RZ};
+        block_partials<2>(v, part, sl, b);
+        return;
+    }
     // 16-byte accesses over the full vectors, then the n % W tail
     const int64_t nv = n / W;
     const Sweep w = xcd_sweep(nv, VB, b);
@@ -1148,11 +1059,11 @@ __global__ __launch_bounds__(VB) void k_update_xr(int64_t n, TX* __restrict__ x,
 // tolerance, the next iteration is a replacement: every block folds its rows
 // of x32 into x64 here and the leader sets rep_at.  At the replacement
 // iteration K3 restarts the direction if K2 asked for it.
-template <typename TX, typename TD>
+template <typename TX, typename TD, int SD = 0>
 __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
                                      const TX* __restrict__ r, const TD* __restrict__ dinv,
                                      const double* part, int g, Scal* sc, int it,
-                                     double* __restrict__ x64, TX* __restrict__ x)
+                                     double* __restrict__ x64, TX* __restrict__ x, int sl_seg = 0)
 {
     typedef typename V16<TX>::type VT;
     constexpr int W = V16<TX>::W;
@@ -1175,6 +1086,10 @@ __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
     }
     if (it == rep_at) {
         if (!restart || done) return;
+        if constexpr (SD > 0) {
+            seg_items<SD>(b.id, sl_seg, n, [&](int64_t i) { p[i] = dinv[i] * r[i]; });
+            return;
+        }
         for (int64_t i = w.first + threadIdx.x; i < w.end; i += w.stride) pv[i] = dv[i] * rv[i];
         for (int64_t i = nv * W + (int64_t)b.id * VB + threadIdx.x; i < n; i += (int64_t)b.n * VB)
             p[i] = (TX)dinv[i] * r[i];
@@ -1207,6 +1122,21 @@ __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
     // K2), done here where p is read anyway; then fold x32 into x64 before
     // a replacement, and p = D^-1 r + beta p
     const TX alpha = (TX)alpha_d;
+    if constexpr (SD > 0) {
+        const TX beta = conv ? (TX)0 : (TX)(rz / rho);
+        const bool fold = mixed && (conv || pause);
+        seg_items<SD>(b.id, sl_seg, n, [&](int64_t i) {
+            const TX pi = p[i];
+            const TX xi = x[i] + alpha * pi;
+            if (fold) x64[i] += (double)xi;
+            x[i] = fold ? (TX)0 : xi;
+            if (!conv) {
+                const TX zi = dinv[i] * r[i];
+                p[i] = zi + beta * pi;
+            }
+        });
+        return;
+    }
     if (mixed && (conv || pause)) {
         // every item is read and written by one thread in one visit (the p
         // update of another thread's item must not precede its x update)
@@ -1256,6 +1186,79 @@ __global__ __launch_bounds__(VB) void k_update_p(int64_t n, TX* __restrict__ p,
     update_p_body<TX, TD>(grid_blk(), n, p, r, dinv, part, g, sc, it, x64, x);
 }
 
+// K2 and K3 on segments
+template <int SD, typename TX>
+__global__ __launch_bounds__(RT) void k_seg_xr(int64_t n, int sl, TX* __restrict__ r,
+                                               const TX* __restrict__ q,
+                                               const TX* __restrict__ dinv, double* part, Scal* sc,
+                                               int it)
+{
+    update_xr_body<TX, TX, SD>(Blk{seg_of_block(blockIdx.x, gridDim.x), (int)gridDim.x}, n, nullptr,
+                               r, nullptr, q, dinv, part, (int)gridDim.x, sc, it, sl);
+}
+
+template <int SD, typename TX>
+__global__ __launch_bounds__(RT) void k_seg_p(int64_t n, int sl, TX* __restrict__ p,
+                                              const TX* __restrict__ r,
+                                              const TX* __restrict__ dinv, const double* part,
+                                              Scal* sc, int it, double* x64, TX* x)
+{
+    update_p_body<TX, TX, SD>(Blk{seg_of_block(blockIdx.x, gridDim.x), (int)gridDim.x}, n, p, r,
+                              dinv, part, (int)gridDim.x, sc, it, x64, x, sl);
+}
+
+// K1 on segments of CSR rows (the products and the p.q sums of CsrForm)
+template <int LPR, typename TV, typename TX, typename TVR>
+__global__ __launch_bounds__(RT) void k_seg_csr(int64_t n, int sl_seg,
+                                                const int32_t* __restrict__ rp,
+                                                const int32_t* __restrict__ col,
+                                                const TV* __restrict__ val,
+                                                const TX* __restrict__ p, TX* __restrict__ q,
+                                                double* part, const Scal* sc, int it, Rep<TVR> R)
+{
+    __shared__ TX qs[RT];
+    const Blk b{seg_of_block(blockIdx.x, gridDim.x), (int)gridDim.x};
+    const int sub = threadIdx.x & (LPR - 1), team = threadIdx.x / LPR;
+    const int64_t row0 = (int64_t)b.id * sl_seg * 64;
+    const int64_t left = n - row0, most = (int64_t)sl_seg * 64;
+    const int rows = (int)(left < 0 ? 0 : (left < most ? left : most));
+    if (it == sc->rep_at) {
+        double tt = 0., rz = 0.;
+        for (int i = team; i < rows; i += RT / LPR) {
+            const int64_t row = row0 + i;
+            const double s = csr_row<LPR, TVR, double, double>(row, sub, rp, col, R.val, R.x64);
+            if (sub == 0) {
+                const double ti = R.b[row] - s;
+                tt += ti * ti;
+                const float rf = (float)ti;
+                R.r32[row] = rf;
+                rz += (double)rf * (double)(R.dinv32[row] * rf);
+            }
+        }
+        double v[2] = {tt, rz};
+        const int sl[2] = {P_TT, P_RZ};
+        block_partials<2>(v, part, sl, b);
+        return;
+    }
+    if (sc->done || sc->stop || it == RES_REPLACE) return;
+    for (int i = team; i < rows; i += RT / LPR) {
+        const int32_t e = rp[row0 + i + 1];
+        const TX s = csr_seg_row<LPR, TV, TX>(rp[row0 + i] + sub, e, val,
+                                              [&](int32_t k) { return p[col[k]]; });
+        if (sub == 0) qs[i] = s;
+    }
+    __syncthreads();
+    double v[1] = {0.};
+    if ((int)threadIdx.x < rows) {
+        const int64_t row = row0 + threadIdx.x;
+        const TX qi = qs[threadIdx.x];
+        q[row] = qi;
+        v[0] += (double)p[row] * (double)qi;
+    }
+    const int sl[1] = {P_PQ};
+    block_partials<1>(v, part, sl, b);
+}
+
 // start: x = 0, r = b, p = D^-1 b; partials of b.b and r.z
 template <typename TX, typename TD>
 __global__ __launch_bounds__(VB) void k_init(int64_t n, const double* __restrict__ b,
@@ -1303,6 +1306,7 @@ __global__ __launch_bounds__(VB) void k_init_fin(const double* part, int g, doub
         sc->conv32 = 0;
         sc->nrep = 0;
         sc->rref = t[0];
+        sc->abort = 0;
     }
 }
 
@@ -2375,6 +2379,100 @@ int run_chunk(Ctx* c, int format, const TV* csr_val, const TV* sell_val, TX* x, 
     return INS_OK;
 }
 
+// K1 of a CSR solve on segments; it = RES_REPLACE: the replacement only
+template <typename TV, typename TX, typename TVR>
+int launch_seg_csr_r(Ctx* c, const Seg& g, const TV* val, const TX* p, TX* q, int it,
+                     const TVR* rep_val)
+{
+    const Rep<TVR> R{rep_val, c->sx64, c->sb, c->r32.p, c->sd32, 0};
+    const int64_t n = c->n_active;
+    const int32_t *rp = c->row_ptr.p, *ci = c->col.p;
+    const Scal* sc = c->scal.p;
+    double* part = c->partial.p;
+    const int lpr = pick_lpr(c);
+    if (lpr == 32)
+        INS_TRY(launch_timed(c, k_seg_csr<32, TV, TX, TVR>, g.B, RT, n, g.R, rp, ci, val, p, q, part, sc, it, R));
+    else if (lpr == 16)
+        INS_TRY(launch_timed(c, k_seg_csr<16, TV, TX, TVR>, g.B, RT, n, g.R, rp, ci, val, p, q, part, sc, it, R));
+    else if (lpr == 8)
+        INS_TRY(launch_timed(c, k_seg_csr<8, TV, TX, TVR>, g.B, RT, n, g.R, rp, ci, val, p, q, part, sc, it, R));
+    else
+        INS_TRY(launch_timed(c, k_seg_csr<4, TV, TX, TVR>, g.B, RT, n, g.R, rp, ci, val, p, q, part, sc, it, R));
+    INS_HIP_CHECK(c, hipGetLastError());
+    return INS_OK;
+}
+
+int launch_seg_csr(Ctx* c, const Seg& g, bool mixed, int it)
+{
+    if (!mixed)
+        return launch_seg_csr_r<double, double, double>(c, g, c->val64.p, c->p.p, c->q.p, it,
+                                                        c->val64.p);
+    if (c->matrix_precision != INS_FP64)
+        return launch_seg_csr_r<float, float, float>(c, g, c->val32.p, c->p32.p, c->q32.p, it,
+                                                     c->val32.p);
+    return launch_seg_csr_r<float, float, double>(c, g, c->val32.p, c->p32.p, c->q32.p, it,
+                                                  c->val64.p);
+}
+
+constexpr int RES_ITERS = 512;   // iterations of a resident launch at most
+
+// the segments of a solve (B = 0: the kernels on the whole vectors)
+Seg solve_segments(const Ctx* c, int format)
+{
+    if (format != INS_FMT_CSR) return Seg{};
+    return csr_segments(c->n_active, lpr_for(c->n_active, c->nnz), c->n_cu);
+}
+
+int resident_fits(Ctx* c, const Seg& g, bool mixed, bool* fits)
+{
+    INS_TRY(csr_windows(c, g, mixed ? 4 : 8));
+    *fits = c->res.csr_ok;
+    return INS_OK;
+}
+
+// one round of a resident solve: iterations until the stop, a replacement
+// or `iters`, then the replacement (which does nothing unless it is due)
+int resident_round(Ctx* c, const Seg& g, bool mixed, int iters, int max_it)
+{
+    const int lpr = pick_lpr(c);
+    if (!mixed)
+        return resident_csr<double>(c, g, lpr, c->val64.p, c->sx64, c->r.p, c->p.p, c->q.p,
+                                    c->sd64, iters, max_it);
+    INS_TRY(resident_csr<float>(c, g, lpr, c->val32.p, c->x32.p, c->r32.p, c->p32.p, c->q32.p,
+                                c->sd32, iters, max_it));
+    INS_TRY(launch_seg_csr(c, g, true, RES_REPLACE));
+    k_seg_xr<1, float><<<g.B, RT, 0, c->stream>>>(c->n_active, g.R, c->r32.p, c->q32.p, c->sd32,
+                                                  c->partial.p, c->scal.p, RES_REPLACE);
+    INS_HIP_CHECK(c, hipGetLastError());
+    return INS_OK;
+}
+
+// one chunk of iterations by the segment kernels
+int run_seg_chunk(Ctx* c, const Seg& g, bool mixed, int k, int64_t* it_launched)
+{
+    const int64_t n = c->n_active;
+    for (int i = 0; i < k; i++) {
+        const int it = (int)*it_launched;
+        INS_TRY(launch_seg_csr(c, g, mixed, it));
+        if (mixed) {
+            k_seg_xr<1, float><<<g.B, RT, 0, c->stream>>>(n, g.R, c->r32.p, c->q32.p, c->sd32,
+                                                          c->partial.p, c->scal.p, it);
+            k_seg_p<1, float><<<g.B, RT, 0, c->stream>>>(n, g.R, c->p32.p, c->r32.p, c->sd32,
+                                                         c->partial.p, c->scal.p, it, c->sx64,
+                                                         c->x32.p);
+        } else {
+            k_seg_xr<1, double><<<g.B, RT, 0, c->stream>>>(n, g.R, c->r.p, c->q.p, c->sd64,
+                                                           c->partial.p, c->scal.p, it);
+            k_seg_p<1, double><<<g.B, RT, 0, c->stream>>>(n, g.R, c->p.p, c->r.p, c->sd64,
+                                                          c->partial.p, c->scal.p, it, c->sx64,
+                                                          c->sx64);
+        }
+        (*it_launched)++;
+    }
+    INS_HIP_CHECK(c, hipGetLastError());
+    return INS_OK;
+}
+
 // Symmetric FP32 slices (see SymView): built when the matrix is scalar in
 // the identity row order, the upper column offsets of all slice lists
 // together number at most SYM_MAXU, and the shared list pads the upper
@@ -2913,49 +3011,76 @@ int solve(Ctx* c, int mode, int format, double rtol, int max_it, int* iters, dou
     c->prof_n = 0;
     INS_HIP_CHECK(c, hipEventRecord(c->ev0, c->stream));
     INS_TRY(solve_vectors(c, format, mode, c->stream));
-    int64_t launched = 0;
     const double delta2 = mixed_delta2();
-    if (!mixed) {
-        k_init<double, double><<<gv, VB, 0, c->stream>>>(n, c->sb, c->sx64, c->r.p, c->p.p,
-                                                         c->sd64, c->partial.p);
-        k_init_fin<<<1, VB, 0, c->stream>>>(c->partial.p, (int)gv, rtol * rtol, 0., c->scal.p);
-    } else {
-        INS_HIP_CHECK(c, hipMemsetAsync(c->sx64, 0, n * sizeof(double), c->stream));
-        k_init<float, float><<<gv, VB, 0, c->stream>>>(n, c->sb, c->x32.p, c->r32.p, c->p32.p,
-                                                       c->sd32, c->partial.p);
-        k_init_fin<<<1, VB, 0, c->stream>>>(c->partial.p, (int)gv, rtol * rtol, delta2,
-                                            c->scal.p);
-    }
-    INS_HIP_CHECK(c, hipGetLastError());
-    INS_TRY(read_scal(c));
+    auto init = [&]() -> int {
+        if (!mixed) {
+            k_init<double, double><<<gv, VB, 0, c->stream>>>(n, c->sb, c->sx64, c->r.p, c->p.p,
+                                                             c->sd64, c->partial.p);
+            k_init_fin<<<1, VB, 0, c->stream>>>(c->partial.p, (int)gv, rtol * rtol, 0., c->scal.p);
+        } else {
+            INS_HIP_CHECK(c, hipMemsetAsync(c->sx64, 0, n * sizeof(double), c->stream));
+            k_init<float, float><<<gv, VB, 0, c->stream>>>(n, c->sb, c->x32.p, c->r32.p, c->p32.p,
+                                                           c->sd32, c->partial.p);
+            k_init_fin<<<1, VB, 0, c->stream>>>(c->partial.p, (int)gv, rtol * rtol, delta2,
+                                                c->scal.p);
+        }
+        INS_HIP_CHECK(c, hipGetLastError());
+        return INS_OK;
+    };
+    INS_TRY(init());
     // The device decides everything, replacements included; the host keeps
     // two chunks queued and stops queueing once a snapshot shows the stop.
     // The iteration limit counts SpMV iterations (replacement iterations,
     // one per replacement, come on top).
     Pipe pipe{c};
-    bool stop = c->h_scal->done != 0;
-    int reps_seen = 0;
-    while (!stop) {
-        while (pipe.inflight < 2 && pipe.enq < max_it + reps_seen) {
-            const int k = std::min(chunk, max_it + reps_seen - pipe.enq);
-            if (mixed)
-                INS_TRY((run_chunk<float, float>(c, format, c->val32.p,
-                                                 format == INS_FMT_SELL ? c->sell.v32.p : nullptr,
-                                                 c->x32.p, c->r32.p, c->p32.p, c->q32.p,
-                                                 c->sd32, k, &launched)));
-            else
-                INS_TRY((run_chunk<double, double>(c, format, c->val64.p,
-                                                   format == INS_FMT_SELL ? c->sell.v64.p : nullptr,
-                                                   c->sx64, c->r.p, c->p.p, c->q.p, c->sd64, k,
-                                                   &launched)));
-            pipe.enq += k;
-            INS_TRY(pipe.issue_snapshot());
+    bool finished = false;
+    const Seg seg = solve_segments(c, format);
+    if (seg.B && !c->profiling) {
+        bool fits = false;
+        INS_TRY(resident_fits(c, seg, mixed, &fits));
+        bool gave_up = false;
+        while (fits && !finished && !gave_up) {
+            while (pipe.inflight < 2) {
+                INS_TRY(resident_round(c, seg, mixed, RES_ITERS, max_it));
+                INS_TRY(pipe.issue_snapshot());
+            }
+            Scal S;
+            INS_TRY(pipe.pop(&S));
+            gave_up = S.abort != 0;
+            finished = !gave_up && (S.done || S.stop || S.iters >= max_it);
         }
-        if (pipe.inflight == 0) break;  // iteration limit
-        Scal S;
-        INS_TRY(pipe.pop(&S));
-        reps_seen = S.nrep;
-        if (S.done || S.stop) stop = true;
+        INS_TRY(pipe.drain());
+        if (gave_up) INS_TRY(init());
+    }
+    if (!finished) {
+        INS_TRY(read_scal(c));
+        bool stop = c->h_scal->done != 0;
+        int reps_seen = 0;
+        int64_t launched = 0;
+        while (!stop) {
+            while (pipe.inflight < 2 && pipe.enq < max_it + reps_seen) {
+                const int k = std::min(chunk, max_it + reps_seen - pipe.enq);
+                if (seg.B)
+                    INS_TRY(run_seg_chunk(c, seg, mixed, k, &launched));
+                else if (mixed)
+                    INS_TRY((run_chunk<float, float>(c, format, c->val32.p,
+                                                     format == INS_FMT_SELL ? c->sell.v32.p : nullptr,
+                                                     c->x32.p, c->r32.p, c->p32.p, c->q32.p,
+                                                     c->sd32, k, &launched)));
+                else
+                    INS_TRY((run_chunk<double, double>(c, format, c->val64.p,
+                                                       format == INS_FMT_SELL ? c->sell.v64.p : nullptr,
+                                                       c->sx64, c->r.p, c->p.p, c->q.p, c->sd64, k,
+                                                       &launched)));
+                pipe.enq += k;
+                INS_TRY(pipe.issue_snapshot());
+            }
+            if (pipe.inflight == 0) break;  // iteration limit
+            Scal S;
+            INS_TRY(pipe.pop(&S));
+            reps_seen = S.nrep;
+            if (S.done || S.stop) stop = true;
+        }
     }
     INS_TRY(pipe.drain());
     if (mixed) {
@@ -3734,8 +3859,9 @@ int server_running(Server* sv) { return sv ? sv->nrun : 0; }
 // Allocation-free FP64 CSR solve (ins_solve_csr_noalloc).
 //
 // The Jacobi-PCG of ins_solve(INS_SOLVE_FP64, INS_FMT_CSR) on a CSR system in
-// caller-owned device arrays, with the same kernels, grids and reduction
-// order (the iterates are the bits ins_solve computes for that system).  Its
+// caller-owned device arrays, with the same row products, segments and
+// order of the sums (the iterates are the bits ins_solve computes for that
+// system, by the resident kernel where one fits).  Its
 // scratch -- the device scalars, the block partials, the Jacobi diagonal and
 // the iterates r, p, q -- lives in `scratch`, a static device array of fixed
 // size: the call allocates nothing (no hipMalloc, hipFree, pinned host
@@ -3785,6 +3911,15 @@ void na_spmv(hipStream_t st, unsigned g, int64_t n, const int32_t* rp, const int
 {
     k_spmv_csr<LPR, double, double, double, double><<<g, SB, 0, st>>>(n, rp, col, val, p, q, part,
                                                                        sc, it, R);
+}
+
+template <int LPR>
+void na_seg(hipStream_t st, const Seg& g, int64_t n, const int32_t* rp, const int32_t* col,
+            const double* val, const double* p, double* q, double* part, const Scal* sc, int it,
+            const Rep<double>& R)
+{
+    k_seg_csr<LPR, double, double, double><<<g.B, RT, 0, st>>>(n, g.R, rp, col, val, p, q, part,
+                                                               sc, it, R);
 }
 
 template <int LPR>
@@ -3840,6 +3975,11 @@ int solve_csr_noalloc(int device, void* stream, int64_t n, int64_t nnz, const in
     const int lpr = lpr_for(n, nnz);
     const unsigned g1 = csr_grid(n, lpr);
     const Rep<double> R{val, x, b, nullptr, nullptr};   // FP64: no replacement
+    int n_cu = 0;
+    if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return INS_ERR_HIP;
+    // the segments ins_solve would take: its resident kernel has these bits
+    const Seg seg = csr_segments(n, lpr, n_cu);
     k_na_dinv<<<grid_for(n, 256), 256, 0, st>>>(n, rp, col, val, dinv);
     k_init<double, double><<<gv, VB, 0, st>>>(n, b, x, r, p, dinv, part);
     k_init_fin<<<1, VB, 0, st>>>(part, (int)gv, rtol * rtol, 0., sc);
@@ -3851,6 +3991,15 @@ int solve_csr_noalloc(int device, void* stream, int64_t n, int64_t nnz, const in
         const int k = std::min(CHUNK, max_it - enq);
         for (int i = 0; i < k; i++) {
             const int it = enq + i;
+            if (seg.B) {
+                if (lpr == 32) na_seg<32>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
+                else if (lpr == 16) na_seg<16>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
+                else if (lpr == 8) na_seg<8>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
+                else na_seg<4>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
+                k_seg_xr<1, double><<<seg.B, RT, 0, st>>>(n, seg.R, r, q, dinv, part, sc, it);
+                k_seg_p<1, double><<<seg.B, RT, 0, st>>>(n, seg.R, p, r, dinv, part, sc, it, x, x);
+                continue;
+            }
             if (lpr == 32) na_spmv<32>(st, g1, n, rp, col, val, p, q, part, sc, it, R);
             else if (lpr == 16) na_spmv<16>(st, g1, n, rp, col, val, p, q, part, sc, it, R);
             else if (lpr == 8) na_spmv<8>(st, g1, n, rp, col, val, p, q, part, sc, it, R);

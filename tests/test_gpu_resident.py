@@ -1,0 +1,116 @@
+"""Resident conjugate gradients (many iterations in one launch, the blocks
+meeting through device-wide sums) against the segment kernels (three launches
+per iteration on the same segments): the same bits, iteration counts and
+residuals.  A profiled solve takes the segment kernels."""
+import json
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from insilico_amd import abi, problems as P
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _banded(n, half, seed):
+    """symmetric, diagonally dominant CSR with up to 2 * half + 1 entries a
+    row at scattered offsets"""
+    r = np.random.RandomState(seed)
+    off = np.unique(np.concatenate([[1], r.randint(1, max(2, n // 2), half)]))[:half]
+    off = off[off < n]
+    row, col, val = [np.arange(n)], [np.arange(n)], [np.full(n, 2.0 * half + 2.0)]
+    for d in off:
+        v = -r.uniform(0.2, 1.0, n - d)
+        i = np.arange(n - d)
+        row += [i, i + d]
+        col += [i + d, i]
+        val += [v, v]
+    row, col, val = np.concatenate(row), np.concatenate(col), np.concatenate(val)
+    o = np.lexsort((col, row))
+    rp = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(row, minlength=n), out=rp[1:])
+    return rp, col[o].astype(np.int32), val[o], r.standard_normal(n)
+
+
+# rows about the edges of slices, of segments (1024 rows for short rows, 512,
+# 256) and of what a window's bitmap holds; row lengths for 4, 8 and 16 lanes,
+# register passes and streamed rows
+CSR = [(1, 1), (2, 1), (63, 2), (64, 2), (65, 2), (1023, 3), (1024, 3), (1025, 3), (4097, 4),
+       (511, 9), (513, 9), (5000, 13), (70001, 13), (140000, 10), (700, 30), (4096, 40),
+       (262144, 2), (262145, 2)]
+
+
+@pytest.mark.parametrize("n,half", CSR)
+def test_csr_resident_equals_segment_kernels(oracle, n, half):
+    print("case", n, half, flush=True)
+    rp, ci, val, b = _banded(n, half, n + half)
+    with abi.Context(0) as c:
+        c.set_csr(rp, ci, val)
+        c.set_rhs(b)
+        for mode in (abi.SOLVE_FP64, abi.SOLVE_MIXED):
+            got = []
+            for prof in (0, 1, 0):
+                c.set_profiling(prof)
+                it, rel, _ = c.solve(mode, abi.FMT_CSR, 1e-9)
+                got.append((it, rel, c.get_solution()))
+            for g in got[1:]:
+                assert g[:2] == got[0][:2]
+                assert np.array_equal(g[2], got[0][2])
+            # the residual is FP64 and of this matrix: what rounding allows
+            r = b - oracle.spmv(rp, ci, val, got[0][2])
+            assert np.linalg.norm(r) <= 1.001e-9 * np.linalg.norm(b) + 1e-13
+
+
+def test_csr_iteration_limit_and_breakdown():
+    rp, ci, val, b = _banded(3000, 4, 5)
+    with abi.Context(0) as c:
+        c.set_csr(rp, ci, val)
+        c.set_rhs(b)
+        for mode in (abi.SOLVE_FP64, abi.SOLVE_MIXED):
+            x = []
+            for prof in (0, 1):
+                c.set_profiling(prof)
+                it, rel, st = c.solve(mode, abi.FMT_CSR, 1e-14, max_it=3, check=False)
+                assert it == 3 and st == abi.ERRORS_INV["NOCONV"]
+                x.append(c.get_solution())
+            assert np.array_equal(x[0], x[1])
+        c.set_profiling(0)
+        c.set_rhs(np.zeros(3000))
+        it, rel, st = c.solve(abi.SOLVE_FP64, abi.FMT_CSR, 1e-9)
+        assert it == 0 and rel == 0.0 and not c.get_solution().any()
+        c.set_csr(rp, ci, -val)
+        c.set_rhs(b)
+        it, rel, st = c.solve(abi.SOLVE_FP64, abi.FMT_CSR, 1e-9, check=False)
+        assert st == abi.ERRORS_INV["BREAKDOWN"]
+
+
+RUN = r"""
+import hashlib, json
+from insilico_amd import abi, problems as P
+out = {}
+with abi.Context(0) as c:
+    c.load_problem(P.diffusion3d(20, seed=3))
+    c.assemble(abi.FP64)
+    for name, mode, fmt in (("fp64 csr", 0, 0), ("mixed csr", 1, 0)):
+        it, rr, _ = c.solve(mode, fmt, 1e-9)
+        out[name] = [it, rr, hashlib.sha256(c.get_solution().tobytes()).hexdigest()]
+print(json.dumps(out), flush=True)
+"""
+
+
+def test_a_wait_that_is_given_up_falls_back():
+    """with a bound of no polls a block gives up at once; the solve is then
+    repeated by the segment kernels, with the same result"""
+    got = []
+    for polls in ("500000", "0"):
+        env = dict(os.environ, INS_RESIDENT_POLLS=polls)
+        r = subprocess.run([sys.executable, "-c", RUN], cwd=ROOT, env=env, capture_output=True,
+                           text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(json.loads(r.stdout.strip().splitlines()[-1]))
+    assert got[0] == got[1]
