@@ -81,8 +81,11 @@ static void release_all(Ctx* c)
     release(c, c->sell.vs64); release(c, c->sell.spw); release(c, c->sell.anode);
     release(c, c->sell.vs); release(c, c->sell.su); release(c, c->sell.smap);
     release(c, c->emask);
-    release(c, c->res.words); release(c, c->res.wlen); release(c, c->res.woff);
-    release(c, c->res.own0); release(c, c->res.wlist); release(c, c->res.lcol);
+    for (WinList* w : {&c->res.csr, &c->res.sell}) {
+        release(c, w->wlen); release(c, w->woff); release(c, w->own0); release(c, w->list);
+    }
+    release(c, c->res.words); release(c, c->res.lcol); release(c, c->res.sell_base);
+    release(c, c->res.cut); release(c, c->res.rel_piece); release(c, c->res.rel_sh);
 }
 
 // A context detached from a server may still be named by the batched work

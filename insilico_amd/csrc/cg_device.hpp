@@ -157,4 +157,13 @@ __device__ inline void load4(const TV* p, TV (&o)[4])
     }
 }
 
+struct SellView {
+    const int32_t* perm;   // slice row -> matrix row (null: identity)
+    const int64_t* sptr;   // value offset of every slice
+    const int32_t* spat;   // column-offset list (pattern) of every slice
+    const int32_t* pptr;
+    const int32_t* plen;
+    const int32_t* pdel;
+};
+
 }  // namespace ins

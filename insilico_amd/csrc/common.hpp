@@ -72,10 +72,6 @@ struct Scal {
                      // solve is to be repeated by the segment kernels
 };
 
-// rep_at of a resident solve: the replacement comes next, whatever the
-// iteration (also the iteration index its kernels are launched with)
-constexpr int RES_REPLACE = INT32_MAX - 1;
-
 // SELL-64 matrix: 64-row slices, values column-major inside a slice; every
 // slice uses one column-offset list (col = row + delta) from a dictionary.
 struct Sell {
@@ -108,6 +104,7 @@ struct Sell {
     bool zeros = false;      // vs sized and zeroed
     int nu = 0;
     DArr<int32_t> su;        // nu offsets, ascending
+    std::vector<int32_t> su_host;
     DArr<float> vs;
     DArr<int32_t> smap;      // nnz: vs position of every CSR entry (-1 below the diagonal)
     int64_t nvs = 0;
@@ -140,17 +137,30 @@ struct Sell {
     DArr<int32_t> anode;
 };
 
+// Windows of a segmentation as lists of columns
+struct WinList {
+    uint64_t gen = 0;        // pattern they were built for
+    int B = 0, R = 0;
+    int wmax = 0, maxlen = 0;   // largest window, longest row or slice
+    DArr<int32_t> wlen, woff, own0, list;
+};
+
 // Segments and windows of the resident solves (resident.hpp)
 struct Resident {
-    DArr<uint64_t> words;    // device-wide sums
-    uint32_t epoch = 0;      // of the next sum
-    // windows of the CSR pattern csr_gen
-    uint64_t csr_gen = 0;
-    int csr_seg_B = 0, csr_seg_R = 0;
-    bool csr_ok = false;
-    int csr_wmax = 0, csr_maxlen = 0;
-    DArr<int32_t> wlen, woff, own0, wlist;
+    DArr<uint64_t> words;    // device-wide sums and the last epoch used
+    int64_t used = 0;        // epochs used at most
+    WinList csr, sell;       // windows of the CSR rows, of the full slices
     DArr<uint16_t> lcol;     // place of every CSR entry's column in its window
+    DArr<int32_t> sell_base; // place of lane 0's column of every slice entry
+    // cuts of the full slices into segments
+    uint64_t cut_gen = 0;
+    int cut_B = 0, cut_R = 0;
+    DArr<int32_t> cut;
+    // the common window of the symmetric slices for segments of rel_R slices
+    uint64_t rel_gen = 0;
+    int rel_R = 0, rel_w = 0, rel_n = 0;
+    DArr<int4> rel_piece;
+    DArr<int32_t> rel_sh;
 };
 
 struct Ctx {

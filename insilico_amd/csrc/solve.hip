@@ -41,6 +41,15 @@
 
 namespace ins {
 
+// mixed: a replacement restarts the direction when |b - A x|^2 exceeds this
+// multiple of the recursive |r|^2 (INS_RESTART_RATIO)
+double restart_ratio()
+{
+    const char* v = std::getenv("INS_RESTART_RATIO");
+    static const double d = (v && *v) ? std::atof(v) : 64.;
+    return d;
+}
+
 namespace {
 
 constexpr int CHUNK = 32;     // FP64 iterations between host checks
@@ -95,15 +104,6 @@ __device__ inline Sweep xcd_sweep(int64_t total, int64_t step, Blk b = grid_blk(
 
 // ---------------------------------------------------------------------------
 // SpMV rows
-struct SellView {
-    const int32_t* perm;   // slice row -> matrix row (null: identity)
-    const int64_t* sptr;   // value offset of every slice
-    const int32_t* spat;   // column-offset list (pattern) of every slice
-    const int32_t* pptr;
-    const int32_t* plen;
-    const int32_t* pdel;
-};
-
 // Values of a slice are stored in groups of 4 consecutive entries per row:
 // position = slice_base + (k/4)*256 + lane*4 + k%4, so a lane reads 4 entries
 // of its row with one 16-byte load (32 bytes for FP64) and a wavefront reads
@@ -924,14 +924,14 @@ struct V16<double> {
 
 // K2: alpha from the p.q partials; r -= alpha q; r.r, r.z partials (the
 // x update waits for K3)
-// SD > 0: on the segments of resident.hpp instead (b.id: the segment, sl: its
+// SD > 0: on the segments of resident.hpp instead (b.id: the segment, seg: its
 // slices, SD components of n items), the items and sums of the resident
 // kernel
 template <typename TX, typename TD, int SD = 0>
 __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* __restrict__ r,
                                       const TX* __restrict__ p, const TX* __restrict__ q,
                                       const TD* __restrict__ dinv, double* part, int g_pq,
-                                      Scal* sc, int it, int sl_seg = 0)
+                                      Scal* sc, int it, Span seg = Span{0, 0})
 {
     // everything this kernel waits on before its sweep -- the scalars of
     // the last iterations and this thread's share of K1's p.q partials --
@@ -964,17 +964,15 @@ __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* 
                 // true residual; once the FP32 recursion has converged or
                 // drifted, restart from p = D^-1 r
                 sc->restart = (sc->conv32 || t[0] > g_restart_ratio * sc->rr) ? 1 : 0;
-                sc->rho[0] = t[1];
-                sc->rho[1] = t[1];
+                sc->rho[(it + 1) & 1] = t[1];
                 sc->rr = t[0];
                 sc->rref = t[0];
             }
             sc->conv32 = 0;
-            if (it == RES_REPLACE) sc->rep_at = INT_MAX;
         }
         return;
     }
-    if (done || it == RES_REPLACE) return;
+    if (done) return;
     if (stop) {
         // converged in the last K3: done from here on
         if (leader(b)) sc->done = 1;
@@ -1002,7 +1000,7 @@ __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* 
     const TX alpha = (TX)ad;
     double rr = 0., rz = 0.;
     if constexpr (SD > 0) {
-        seg_items<SD>(b.id, sl_seg, n, [&](int64_t i) {
+        seg_items<SD>(seg, n, [&](int64_t i) {
             const TX ri = r[i] - alpha * q[i];
             r[i] = ri;
             const TX zi = dinv[i] * ri;
@@ -1063,7 +1061,8 @@ template <typename TX, typename TD, int SD = 0>
 __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
                                      const TX* __restrict__ r, const TD* __restrict__ dinv,
                                      const double* part, int g, Scal* sc, int it,
-                                     double* __restrict__ x64, TX* __restrict__ x, int sl_seg = 0)
+                                     double* __restrict__ x64, TX* __restrict__ x,
+                                     Span seg = Span{0, 0})
 {
     typedef typename V16<TX>::type VT;
     constexpr int W = V16<TX>::W;
@@ -1087,7 +1086,7 @@ __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
     if (it == rep_at) {
         if (!restart || done) return;
         if constexpr (SD > 0) {
-            seg_items<SD>(b.id, sl_seg, n, [&](int64_t i) { p[i] = dinv[i] * r[i]; });
+            seg_items<SD>(seg, n, [&](int64_t i) { p[i] = dinv[i] * r[i]; });
             return;
         }
         for (int64_t i = w.first + threadIdx.x; i < w.end; i += w.stride) pv[i] = dv[i] * rv[i];
@@ -1125,7 +1124,7 @@ __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
     if constexpr (SD > 0) {
         const TX beta = conv ? (TX)0 : (TX)(rz / rho);
         const bool fold = mixed && (conv || pause);
-        seg_items<SD>(b.id, sl_seg, n, [&](int64_t i) {
+        seg_items<SD>(seg, n, [&](int64_t i) {
             const TX pi = p[i];
             const TX xi = x[i] + alpha * pi;
             if (fold) x64[i] += (double)xi;
@@ -1188,23 +1187,24 @@ __global__ __launch_bounds__(VB) void k_update_p(int64_t n, TX* __restrict__ p,
 
 // K2 and K3 on segments
 template <int SD, typename TX>
-__global__ __launch_bounds__(RT) void k_seg_xr(int64_t n, int sl, TX* __restrict__ r,
+__global__ __launch_bounds__(RT) void k_seg_xr(int64_t n, Seg g, TX* __restrict__ r,
                                                const TX* __restrict__ q,
                                                const TX* __restrict__ dinv, double* part, Scal* sc,
                                                int it)
 {
-    update_xr_body<TX, TX, SD>(Blk{seg_of_block(blockIdx.x, gridDim.x), (int)gridDim.x}, n, nullptr,
-                               r, nullptr, q, dinv, part, (int)gridDim.x, sc, it, sl);
+    const Blk b{seg_of_block(blockIdx.x, g.B), g.B};
+    update_xr_body<TX, TX, SD>(b, n, nullptr, r, nullptr, q, dinv, part, g.B, sc, it,
+                               seg_span(g, b.id));
 }
 
 template <int SD, typename TX>
-__global__ __launch_bounds__(RT) void k_seg_p(int64_t n, int sl, TX* __restrict__ p,
+__global__ __launch_bounds__(RT) void k_seg_p(int64_t n, Seg g, TX* __restrict__ p,
                                               const TX* __restrict__ r,
                                               const TX* __restrict__ dinv, const double* part,
                                               Scal* sc, int it, double* x64, TX* x)
 {
-    update_p_body<TX, TX, SD>(Blk{seg_of_block(blockIdx.x, gridDim.x), (int)gridDim.x}, n, p, r,
-                              dinv, part, (int)gridDim.x, sc, it, x64, x, sl);
+    const Blk b{seg_of_block(blockIdx.x, g.B), g.B};
+    update_p_body<TX, TX, SD>(b, n, p, r, dinv, part, g.B, sc, it, x64, x, seg_span(g, b.id));
 }
 
 // K1 on segments of CSR rows (the products and the p.q sums of CsrForm)
@@ -1216,7 +1216,7 @@ __global__ __launch_bounds__(RT) void k_seg_csr(int64_t n, int sl_seg,
                                                 const TX* __restrict__ p, TX* __restrict__ q,
                                                 double* part, const Scal* sc, int it, Rep<TVR> R)
 {
-    __shared__ TX qs[RT];
+    __shared__ TX qs[CSR_ROWS];
     const Blk b{seg_of_block(blockIdx.x, gridDim.x), (int)gridDim.x};
     const int sub = threadIdx.x & (LPR - 1), team = threadIdx.x / LPR;
     const int64_t row0 = (int64_t)b.id * sl_seg * 64;
@@ -1240,7 +1240,7 @@ __global__ __launch_bounds__(RT) void k_seg_csr(int64_t n, int sl_seg,
         block_partials<2>(v, part, sl, b);
         return;
     }
-    if (sc->done || sc->stop || it == RES_REPLACE) return;
+    if (sc->done || sc->stop) return;
     for (int i = team; i < rows; i += RT / LPR) {
         const int32_t e = rp[row0 + i + 1];
         const TX s = csr_seg_row<LPR, TV, TX>(rp[row0 + i] + sub, e, val,
@@ -1249,14 +1249,63 @@ __global__ __launch_bounds__(RT) void k_seg_csr(int64_t n, int sl_seg,
     }
     __syncthreads();
     double v[1] = {0.};
-    if ((int)threadIdx.x < rows) {
-        const int64_t row = row0 + threadIdx.x;
-        const TX qi = qs[threadIdx.x];
-        q[row] = qi;
-        v[0] += (double)p[row] * (double)qi;
+    for (int i = threadIdx.x; i < rows; i += RT) {
+        const TX qi = qs[i];
+        q[row0 + i] = qi;
+        v[0] += (double)p[row0 + i] * (double)qi;
     }
     const int sl[1] = {P_PQ};
     block_partials<1>(v, part, sl, b);
+}
+
+// K1 on a segment of a SELL storage (at the replacement iteration the FP64
+// residual)
+template <int F, typename TV, typename TX, typename TVR>
+__device__ inline void seg_spmv_body(Blk b, const Span& sp, int64_t n, const SellView& S,
+                                     const int32_t* __restrict__ u, const TV* __restrict__ vals,
+                                     const TX* __restrict__ p, TX* __restrict__ q, double* part,
+                                     const Scal* sc, int it, const Rep<TVR>& R, double* lds)
+{
+    if (it == sc->rep_at) {
+        double v[2] = {0., 0.};
+        seg_products<F, TVR, double>(sp, n, S, u, R.val, [&](int i) { return R.x64[i]; },
+                                     lds, [&](int g, double s) {
+                                         const double ti = R.b[g] - s;
+                                         v[0] += ti * ti;
+                                         const float rf = (float)ti;
+                                         R.r32[g] = rf;
+                                         v[1] += (double)rf * (double)(R.dinv32[g] * rf);
+                                     });
+        const int slot[2] = {P_TT, P_RZ};
+        block_partials<2>(v, part, slot, b);
+        return;
+    }
+    if (sc->done || sc->stop) return;
+    double v[1] = {0.};
+    seg_products<F, TV, TX>(sp, n, S, u, vals, [&](int i) { return p[i]; },
+                            reinterpret_cast<TX*>(lds), [&](int g, TX s) {
+                                q[g] = s;
+                                v[0] += (double)p[g] * (double)s;
+                            });
+    const int slot[1] = {P_PQ};
+    block_partials<1>(v, part, slot, b);
+}
+
+constexpr int form_parts_lds(int F)
+{
+    return F == SEG_BSYM3 ? BSYM_TASKS * 3 * 64 : (F == SEG_BSYM2 ? BSYM_TASKS * 2 * 64 : 1);
+}
+
+template <int F, typename TV, typename TX, typename TVR>
+__global__ __launch_bounds__(RT) void k_seg_sell(int64_t n, Seg g, SellView S,
+                                                 const int32_t* __restrict__ u,
+                                                 const TV* __restrict__ vals,
+                                                 const TX* __restrict__ p, TX* __restrict__ q,
+                                                 double* part, const Scal* sc, int it, Rep<TVR> R)
+{
+    __shared__ double lds[form_parts_lds(F)];
+    const Blk b{seg_of_block(blockIdx.x, g.B), g.B};
+    seg_spmv_body<F, TV, TX, TVR>(b, seg_span(g, b.id), n, S, u, vals, p, q, part, sc, it, R, lds);
 }
 
 // start: x = 0, r = b, p = D^-1 b; partials of b.b and r.z
@@ -2069,7 +2118,7 @@ int ensure_solver_state(Ctx* c, int mode)
         INS_HIP_CHECK(c, hipMemcpyToSymbol(HIP_SYMBOL(g_nt), &nt, sizeof(int)));
         const int bands = env_int("INS_BSYM_BANDS", 4);
         INS_HIP_CHECK(c, hipMemcpyToSymbol(HIP_SYMBOL(g_bsym_bands), &bands, sizeof(int)));
-        const double ratio = env_double("INS_RESTART_RATIO", 64.);
+        const double ratio = restart_ratio();
         INS_HIP_CHECK(c, hipMemcpyToSymbol(HIP_SYMBOL(g_restart_ratio), &ratio, sizeof(double)));
     }
     for (int i = 0; i < 2; i++)
@@ -2379,7 +2428,7 @@ int run_chunk(Ctx* c, int format, const TV* csr_val, const TV* sell_val, TX* x, 
     return INS_OK;
 }
 
-// K1 of a CSR solve on segments; it = RES_REPLACE: the replacement only
+// K1 of a CSR solve on segments
 template <typename TV, typename TX, typename TVR>
 int launch_seg_csr_r(Ctx* c, const Seg& g, const TV* val, const TX* p, TX* q, int it,
                      const TVR* rep_val)
@@ -2414,62 +2463,157 @@ int launch_seg_csr(Ctx* c, const Seg& g, bool mixed, int it)
                                                   c->val64.p);
 }
 
-constexpr int RES_ITERS = 512;   // iterations of a resident launch at most
+constexpr int RES_ITERS = 2048;   // iterations of a resident launch at most
 
-// the segments of a solve (B = 0: the kernels on the whole vectors)
-Seg solve_segments(const Ctx* c, int format)
-{
-    if (format != INS_FMT_CSR) return Seg{};
-    return csr_segments(c->n_active, lpr_for(c->n_active, c->nnz), c->n_cu);
-}
+// A solve's segments (B = 0: the kernels on the whole vectors) and their form
+struct SegSolve {
+    Seg g;
+    int format = INS_FMT_CSR;
+    SegForm form = SEG_NONE;
+    int D = 1;          // components per item
+    int64_t items = 0;
+    bool mixed = false;
+};
 
-int resident_fits(Ctx* c, const Seg& g, bool mixed, bool* fits)
+int solve_segments(Ctx* c, int format, bool mixed, SegSolve* s)
 {
-    INS_TRY(csr_windows(c, g, mixed ? 4 : 8));
-    *fits = c->res.csr_ok;
+    s->format = format;
+    s->mixed = mixed;
+    s->items = c->n_active;
+    if (format == INS_FMT_CSR) {
+        s->g = csr_segments(c->n_active, lpr_for(c->n_active, c->nnz), c->n_cu, mixed);
+        return INS_OK;
+    }
+    const int st = sell_segments(c, mixed, &s->g);
+    if (st == INS_ERR_OOM) s->g = Seg{};   // no memory for windows: the plain kernels
+    else INS_TRY(st);
+    s->form = sell_form(c);
+    s->D = s->form == SEG_BSYM3 ? 3 : (s->form == SEG_BSYM2 ? 2 : 1);
+    if (s->D > 1) s->items = c->sell.snodes;
     return INS_OK;
 }
 
-// one round of a resident solve: iterations until the stop, a replacement
-// or `iters`, then the replacement (which does nothing unless it is due)
-int resident_round(Ctx* c, const Seg& g, bool mixed, int iters, int max_it)
+template <int F, typename TV, typename TX, typename TVR>
+int launch_seg_sell_f(Ctx* c, const SegSolve& s, const TV* val, const TX* p, TX* q, int it,
+                      const TVR* rep_val)
 {
-    const int lpr = pick_lpr(c);
-    if (!mixed)
-        return resident_csr<double>(c, g, lpr, c->val64.p, c->sx64, c->r.p, c->p.p, c->q.p,
-                                    c->sd64, iters, max_it);
-    INS_TRY(resident_csr<float>(c, g, lpr, c->val32.p, c->x32.p, c->r32.p, c->p32.p, c->q32.p,
-                                c->sd32, iters, max_it));
-    INS_TRY(launch_seg_csr(c, g, true, RES_REPLACE));
-    k_seg_xr<1, float><<<g.B, RT, 0, c->stream>>>(c->n_active, g.R, c->r32.p, c->q32.p, c->sd32,
-                                                  c->partial.p, c->scal.p, RES_REPLACE);
+    const Rep<TVR> R{rep_val, c->sx64, c->sb, c->r32.p, c->sd32, 0};
+    const Scal* sc = c->scal.p;
+    INS_TRY(launch_timed(c, k_seg_sell<F, TV, TX, TVR>, s.g.B, RT, s.items, s.g, sell_view(c),
+                         (const int32_t*)c->sell.su.p, val, p, q, c->partial.p, sc, it, R));
     INS_HIP_CHECK(c, hipGetLastError());
     return INS_OK;
+}
+
+template <typename TV, typename TX, typename TVR>
+int launch_seg_sell_r(Ctx* c, const SegSolve& s, const TV* sym, const TV* full, const TX* p, TX* q,
+                      int it, const TVR* rep_sym, const TVR* rep_full)
+{
+    switch (s.form) {
+    case SEG_SYM14: return launch_seg_sell_f<SEG_SYM14, TV, TX, TVR>(c, s, sym, p, q, it, rep_sym);
+    case SEG_SYM5: return launch_seg_sell_f<SEG_SYM5, TV, TX, TVR>(c, s, sym, p, q, it, rep_sym);
+    case SEG_BSYM3: return launch_seg_sell_f<SEG_BSYM3, TV, TX, TVR>(c, s, sym, p, q, it, rep_sym);
+    case SEG_BSYM2: return launch_seg_sell_f<SEG_BSYM2, TV, TX, TVR>(c, s, sym, p, q, it, rep_sym);
+    default: return launch_seg_sell_f<SEG_SELL, TV, TX, TVR>(c, s, full, p, q, it, rep_full);
+    }
+}
+
+// K1 of a solve on segments
+int launch_seg_spmv(Ctx* c, const SegSolve& s, int it)
+{
+    if (s.format == INS_FMT_CSR) return launch_seg_csr(c, s.g, s.mixed, it);
+    const Sell& L = c->sell;
+    if (!s.mixed)
+        return launch_seg_sell_r<double, double, double>(c, s, L.vs64.p, L.v64.p, c->p.p, c->q.p,
+                                                         it, L.vs64.p, L.v64.p);
+    if (c->matrix_precision != INS_FP64)
+        return launch_seg_sell_r<float, float, float>(c, s, L.vs.p, L.v32.p, c->p32.p, c->q32.p,
+                                                      it, L.vs.p, L.v32.p);
+    return launch_seg_sell_r<float, float, double>(c, s, L.vs.p, L.v32.p, c->p32.p, c->q32.p, it,
+                                                   L.vs64.p, L.v64.p);
+}
+
+template <typename T>
+int launch_seg_xr(Ctx* c, const SegSolve& s, T* r, const T* q, const T* dinv, int it)
+{
+    if (s.D == 3)
+        k_seg_xr<3, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
+    else if (s.D == 2)
+        k_seg_xr<2, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
+    else
+        k_seg_xr<1, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
+    INS_HIP_CHECK(c, hipGetLastError());
+    return INS_OK;
+}
+
+template <typename T>
+int launch_seg_p(Ctx* c, const SegSolve& s, T* p, const T* r, const T* dinv, T* x, int it)
+{
+    if (s.D == 3)
+        k_seg_p<3, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+    else if (s.D == 2)
+        k_seg_p<2, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+    else
+        k_seg_p<1, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+    INS_HIP_CHECK(c, hipGetLastError());
+    return INS_OK;
+}
+
+// windows and words of a resident solve; no memory for them: not resident
+int resident_fits(Ctx* c, const SegSolve& s, bool* fits)
+{
+    *fits = false;
+    if (!s.g.B) return INS_OK;
+    const int vb = s.mixed ? 4 : 8;
+    int st = s.format == INS_FMT_CSR ? csr_windows(c, s.g, vb, fits)
+                                     : sell_windows(c, s.g, vb, fits);
+    if (st == INS_OK && *fits) st = resident_words(c, c->stream, 0);
+    if (st == INS_ERR_OOM) *fits = false;
+    return st == INS_ERR_OOM ? INS_OK : st;
+}
+
+// up to RES_ITERS iterations of a resident solve, replacements included
+int resident_launch(Ctx* c, const SegSolve& s, int max_it)
+{
+    const bool csr = s.format == INS_FMT_CSR;
+    const bool f64 = c->matrix_precision == INS_FP64;
+    ResRep rep;
+    rep.ratio = restart_ratio();
+    rep.b = c->sb;
+    rep.x64 = c->sx64;
+    const Sell& L = c->sell;
+    const bool sym = s.form != SEG_SELL;
+    rep.v64 = !f64 ? nullptr : csr ? c->val64.p : sym ? L.vs64.p : L.v64.p;
+    rep.v32 = f64 ? nullptr : csr ? c->val32.p : sym ? L.vs.p : L.v32.p;
+    if (s.mixed) {
+        if (csr)
+            return resident_csr<float>(c, s.g, pick_lpr(c), c->val32.p, c->x32.p, c->r32.p,
+                                       c->p32.p, c->q32.p, c->sd32, rep, RES_ITERS, max_it);
+        return resident_sell<float>(c, s.g, c->x32.p, c->r32.p, c->p32.p, c->q32.p, c->sd32, rep,
+                                    RES_ITERS, max_it);
+    }
+    if (csr)
+        return resident_csr<double>(c, s.g, pick_lpr(c), c->val64.p, c->sx64, c->r.p, c->p.p,
+                                    c->q.p, c->sd64, rep, RES_ITERS, max_it);
+    return resident_sell<double>(c, s.g, c->sx64, c->r.p, c->p.p, c->q.p, c->sd64, rep, RES_ITERS,
+                                 max_it);
 }
 
 // one chunk of iterations by the segment kernels
-int run_seg_chunk(Ctx* c, const Seg& g, bool mixed, int k, int64_t* it_launched)
+int run_seg_chunk(Ctx* c, const SegSolve& s, int k, int64_t* it_launched)
 {
-    const int64_t n = c->n_active;
     for (int i = 0; i < k; i++) {
         const int it = (int)*it_launched;
-        INS_TRY(launch_seg_csr(c, g, mixed, it));
-        if (mixed) {
-            k_seg_xr<1, float><<<g.B, RT, 0, c->stream>>>(n, g.R, c->r32.p, c->q32.p, c->sd32,
-                                                          c->partial.p, c->scal.p, it);
-            k_seg_p<1, float><<<g.B, RT, 0, c->stream>>>(n, g.R, c->p32.p, c->r32.p, c->sd32,
-                                                         c->partial.p, c->scal.p, it, c->sx64,
-                                                         c->x32.p);
+        INS_TRY(launch_seg_spmv(c, s, it));
+        if (s.mixed) {
+            INS_TRY(launch_seg_xr<float>(c, s, c->r32.p, c->q32.p, c->sd32, it));
+            INS_TRY(launch_seg_p<float>(c, s, c->p32.p, c->r32.p, c->sd32, c->x32.p, it));
         } else {
-            k_seg_xr<1, double><<<g.B, RT, 0, c->stream>>>(n, g.R, c->r.p, c->q.p, c->sd64,
-                                                           c->partial.p, c->scal.p, it);
-            k_seg_p<1, double><<<g.B, RT, 0, c->stream>>>(n, g.R, c->p.p, c->r.p, c->sd64,
-                                                          c->partial.p, c->scal.p, it, c->sx64,
-                                                          c->sx64);
+            INS_TRY(launch_seg_xr<double>(c, s, c->r.p, c->q.p, c->sd64, it));
+            INS_TRY(launch_seg_p<double>(c, s, c->p.p, c->r.p, c->sd64, c->sx64, it));
         }
         (*it_launched)++;
     }
-    INS_HIP_CHECK(c, hipGetLastError());
     return INS_OK;
 }
 
@@ -2594,6 +2738,7 @@ int build_bsym(Ctx* c)
     (void)hipFreeAsync(err, c->stream);
     if (herr) return INS_OK;
     S.nu = nu;
+    S.su_host = up;
     S.nvs = nvs;
     S.sdpn = D;
     S.snodes = N;
@@ -2668,6 +2813,7 @@ int build_sym(Ctx* c)
     (void)hipFreeAsync(err, c->stream);
     if (herr) return INS_OK;
     S.nu = nu;
+    S.su_host = up;
     S.nvs = nvs;
     // stencil lines: {0, 1, c1 - 1, c1, c1 + 1, ...} with 1 < c1 - 1, the
     // centres ascending and every line at least one wave (64 rows) apart
@@ -3034,24 +3180,27 @@ int solve(Ctx* c, int mode, int format, double rtol, int max_it, int* iters, dou
     // one per replacement, come on top).
     Pipe pipe{c};
     bool finished = false;
-    const Seg seg = solve_segments(c, format);
-    if (seg.B && !c->profiling) {
+    SegSolve seg;
+    INS_TRY(solve_segments(c, format, mixed, &seg));
+    if (seg.g.B && !c->profiling) {
         bool fits = false;
-        INS_TRY(resident_fits(c, seg, mixed, &fits));
+        INS_TRY(resident_fits(c, seg, &fits));
         bool gave_up = false;
         while (fits && !finished && !gave_up) {
-            while (pipe.inflight < 2) {
-                INS_TRY(resident_round(c, seg, mixed, RES_ITERS, max_it));
-                INS_TRY(pipe.issue_snapshot());
-            }
-            Scal S;
-            INS_TRY(pipe.pop(&S));
+            INS_TRY(resident_launch(c, seg, max_it));
+            // the last launch as a rule: what follows a solve goes with it
+            if (!mixed) INS_TRY(launch_resid(c, format));
+            INS_TRY(read_scal(c));
+            const Scal& S = *c->h_scal;
             gave_up = S.abort != 0;
             finished = !gave_up && (S.done || S.stop || S.iters >= max_it);
         }
-        INS_TRY(pipe.drain());
-        if (gave_up) INS_TRY(init());
+        if (gave_up) {
+            INS_TRY(resident_reset(c, c->stream));
+            INS_TRY(init());
+        }
     }
+    const bool resident = finished;
     if (!finished) {
         INS_TRY(read_scal(c));
         bool stop = c->h_scal->done != 0;
@@ -3060,8 +3209,8 @@ int solve(Ctx* c, int mode, int format, double rtol, int max_it, int* iters, dou
         while (!stop) {
             while (pipe.inflight < 2 && pipe.enq < max_it + reps_seen) {
                 const int k = std::min(chunk, max_it + reps_seen - pipe.enq);
-                if (seg.B)
-                    INS_TRY(run_seg_chunk(c, seg, mixed, k, &launched));
+                if (seg.g.B)
+                    INS_TRY(run_seg_chunk(c, seg, k, &launched));
                 else if (mixed)
                     INS_TRY((run_chunk<float, float>(c, format, c->val32.p,
                                                      format == INS_FMT_SELL ? c->sell.v32.p : nullptr,
@@ -3084,13 +3233,13 @@ int solve(Ctx* c, int mode, int format, double rtol, int max_it, int* iters, dou
     }
     INS_TRY(pipe.drain());
     if (mixed) {
-        INS_TRY(read_scal(c));
+        if (!resident) INS_TRY(read_scal(c));
         if (!c->h_scal->fin && !c->h_scal->breakdown) {
             // iteration limit: fold what was computed and measure it
             k_fold<<<gv, VB, 0, c->stream>>>(n, c->sx64, c->x32.p);
             INS_TRY(launch_resid(c, format));
         }
-    } else {
+    } else if (!resident) {
         INS_TRY(launch_resid(c, format));
     }
     INS_TRY(solve_vectors_out(c, c->stream));
@@ -3139,6 +3288,12 @@ int prepare(Ctx* c, int mode, int format)
     }
     c->want_format = format;
     INS_TRY(ensure_solver_state(c, mode));
+    if (format == INS_FMT_SELL ? c->sell.ok : c->have_matrix) {
+        SegSolve seg;
+        bool fits;
+        INS_TRY(solve_segments(c, format, mode == INS_SOLVE_MIXED, &seg));
+        INS_TRY(resident_fits(c, seg, &fits));
+    }
     INS_HIP_CHECK(c, hipStreamSynchronize(c->stream));
     return INS_OK;
 }
@@ -3425,6 +3580,9 @@ struct SlotDesc {
     int slines;
     int64_t join;  // batched iteration of the request's first launch
     int g_spmv, g_vec;
+    int form, seg_b, seg_r;   // SegForm and segments (seg_b = 0: none)
+    const int32_t INS_GLOBAL* cut;
+    int64_t items;
 };
 
 __device__ inline SellView sell_of(const GSellView& g)
@@ -3443,6 +3601,8 @@ struct BatchTab {
     int nslot, pad;
     int pre_spmv[MAXS + 1];  // first block of every request in kb_spmv
     int pre_vec[MAXS + 1];   // ... in kb_update_xr / kb_update_p
+    int pre_seg[MAXS + 1];   // ... in the kernels on segments
+    CgEntry cg[MAXS];        // the requests of the resident launches
     SlotDesc d[MAXS];
 };
 
@@ -3493,6 +3653,71 @@ __global__ __launch_bounds__(VB) void kb_update_p(const BatchTab* __restrict__ b
                                 (float*)d.x);
 }
 
+// the same three kernels for the requests that are solved on segments
+__global__ __launch_bounds__(RT) void kb_seg_spmv(const BatchTab* __restrict__ bt, int64_t it)
+{
+    __shared__ double lds[form_parts_lds(SEG_BSYM3)];
+    const int s = find_slot(bt->pre_seg, bt->nslot, blockIdx.x);
+    const SlotDesc& d = bt->d[s];
+    const Rep<double> R{(const double*)d.v64, (const double*)d.x64, (const double*)d.b,
+                        (float*)d.r, (const float*)d.dinv, 0};
+    const Blk b{seg_of_block((int)blockIdx.x - bt->pre_seg[s], d.seg_b), d.seg_b};
+    const SellView S = sell_of(d.S);
+    const int32_t* u = (const int32_t*)d.su;
+    const float* sym = (const float*)d.vs;
+    const float* p = (const float*)d.p;
+    float* q = (float*)d.q;
+    double* part = (double*)d.part;
+    const Scal* sc = (const Scal*)d.sc;
+    const int i = (int)(it - d.join);
+    const Span sp = seg_span(Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, b.id);
+    switch (d.form) {
+    case SEG_SYM14: seg_spmv_body<SEG_SYM14, float, float, double>(b, sp, d.items, S, u, sym, p, q, part, sc, i, R, lds); break;
+    case SEG_SYM5: seg_spmv_body<SEG_SYM5, float, float, double>(b, sp, d.items, S, u, sym, p, q, part, sc, i, R, lds); break;
+    case SEG_BSYM3: seg_spmv_body<SEG_BSYM3, float, float, double>(b, sp, d.items, S, u, sym, p, q, part, sc, i, R, lds); break;
+    case SEG_BSYM2: seg_spmv_body<SEG_BSYM2, float, float, double>(b, sp, d.items, S, u, sym, p, q, part, sc, i, R, lds); break;
+    default: seg_spmv_body<SEG_SELL, float, float, double>(b, sp, d.items, S, u, (const float*)d.val, p, q, part, sc, i, R, lds); break;
+    }
+}
+
+template <int SD>
+__device__ inline void kb_seg_xr_d(const SlotDesc& d, Blk b, int i)
+{
+    update_xr_body<float, float, SD>(b, d.items, (float*)nullptr, (float*)d.r, nullptr,
+                                     (const float*)d.q, (const float*)d.dinv, (double*)d.part,
+                                     d.seg_b, (Scal*)d.sc, i,
+                                     seg_span(Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, b.id));
+}
+__global__ __launch_bounds__(RT) void kb_seg_xr(const BatchTab* __restrict__ bt, int64_t it)
+{
+    const int s = find_slot(bt->pre_seg, bt->nslot, blockIdx.x);
+    const SlotDesc& d = bt->d[s];
+    const Blk b{seg_of_block((int)blockIdx.x - bt->pre_seg[s], d.seg_b), d.seg_b};
+    const int i = (int)(it - d.join);
+    if (d.form == SEG_BSYM3) kb_seg_xr_d<3>(d, b, i);
+    else if (d.form == SEG_BSYM2) kb_seg_xr_d<2>(d, b, i);
+    else kb_seg_xr_d<1>(d, b, i);
+}
+
+template <int SD>
+__device__ inline void kb_seg_p_d(const SlotDesc& d, Blk b, int i)
+{
+    update_p_body<float, float, SD>(b, d.items, (float*)d.p, (const float*)d.r,
+                                    (const float*)d.dinv, (const double*)d.part, d.seg_b,
+                                    (Scal*)d.sc, i, (double*)d.x64, (float*)d.x,
+                                    seg_span(Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, b.id));
+}
+__global__ __launch_bounds__(RT) void kb_seg_p(const BatchTab* __restrict__ bt, int64_t it)
+{
+    const int s = find_slot(bt->pre_seg, bt->nslot, blockIdx.x);
+    const SlotDesc& d = bt->d[s];
+    const Blk b{seg_of_block((int)blockIdx.x - bt->pre_seg[s], d.seg_b), d.seg_b};
+    const int i = (int)(it - d.join);
+    if (d.form == SEG_BSYM3) kb_seg_p_d<3>(d, b, i);
+    else if (d.form == SEG_BSYM2) kb_seg_p_d<2>(d, b, i);
+    else kb_seg_p_d<1>(d, b, i);
+}
+
 }  // namespace
 
 struct SlotH {
@@ -3507,6 +3732,8 @@ struct SlotH {
     int iters = 0;
     double relres = 0.;
     bool relres_known = false;
+    SegSolve seg;   // the segments of its solve (seg.g.B = 0: none)
+    bool resident = false;    // it runs in the resident launches
 };
 
 struct Server {
@@ -3527,10 +3754,15 @@ struct Server {
     int tab_cur = 0;
     bool dirty = true;
     int nrun = 0;
-    int grid_spmv = 0, grid_vec = 0;
+    int grid_spmv = 0, grid_vec = 0, grid_seg = 0;
+    std::vector<CgGroup> groups;
     int64_t it = 0;      // batched iterations launched
     int64_t chunks = 0;  // chunks launched
     hipEvent_t ev_sync = nullptr;
+    // the resident launches of a step that has batched kernels too: those
+    // leave most of every compute unit idle, and the chains are independent
+    hipStream_t side = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 };
 
 namespace {
@@ -3577,13 +3809,43 @@ int finish(Server* sv, int s, int status, const Scal* S)
     return hand_back(sv, h);
 }
 
+// x = 0, r = b, p = D^-1 b and the scalars of a request, on the server stream
+int start_request(Server* sv, int s, Ctx* c, double rtol)
+{
+    const int64_t n = c->n_active;
+    const unsigned gv = vec_grid(n);
+    SRV_HIP(sv, hipMemsetAsync(c->sx64, 0, n * sizeof(double), sv->stream));
+    k_init<float, float><<<gv, VB, 0, sv->stream>>>(n, c->sb, c->x32.p, c->r32.p, c->p32.p,
+                                                    c->sd32, c->partial.p);
+    k_init_fin<<<1, VB, 0, sv->stream>>>(c->partial.p, (int)gv, rtol * rtol, mixed_delta2(),
+                                         sv->scal + s);
+    SRV_HIP(sv, hipGetLastError());
+    return INS_OK;
+}
+
+int restart_on_segments(Server* sv, int s)
+{
+    SlotH& h = sv->slots[s];
+    if (resident_reset(h.c, sv->stream) != INS_OK) return sfail(sv, INS_ERR_HIP, h.c->err);
+    INS_TRY(start_request(sv, s, h.c, h.rtol));
+    h.resident = false;
+    h.join_it = sv->it;
+    h.join_chunk = sv->chunks;
+    sv->dirty = true;
+    return INS_OK;
+}
+
 int process_snapshot(Server* sv, int64_t chunk, const Scal* snap)
 {
     for (int s = 0; s < sv->max_slots; s++) {
         SlotH& h = sv->slots[s];
         if (h.state != INS_SLOT_RUNNING || chunk < h.join_chunk) continue;
         const Scal& S = snap[s];
-        if (S.fin) {
+        if (S.abort && h.resident) {
+            // a wait of the resident launch was given up: again from the
+            // start, by the segment kernels (the same iterates)
+            INS_TRY(restart_on_segments(sv, s));
+        } else if (S.fin) {
             INS_TRY(finish(sv, s, INS_OK, &S));
         } else if (S.breakdown) {
             INS_TRY(finish(sv, s, INS_ERR_BREAKDOWN, &S));
@@ -3607,7 +3869,13 @@ int upload_table(Server* sv)
     const int t = (sv->tab_cur + 1) % Server::NTAB;
     SRV_HIP(sv, hipEventSynchronize(sv->tab_ev[t]));
     BatchTab& T = sv->h_tab[t];
-    int ns = 0, gs = 0, gvv = 0;
+    int ns = 0, gs = 0, gvv = 0, gseg = 0, ncg = 0;
+    sv->groups.clear();
+    // beside batched kernels a resident launch leaves them a quarter of the
+    // compute units (a resident block fills its own): a batch of eight
+    // requests, one of them not resident, took 23.5 ms, 25.3 without
+    bool beside = false;
+    for (const SlotH& h : sv->slots) beside |= h.state == INS_SLOT_RUNNING && !h.resident;
     for (int s = 0; s < sv->max_slots; s++) {
         const SlotH& h = sv->slots[s];
         if (h.state != INS_SLOT_RUNNING) continue;
@@ -3644,17 +3912,41 @@ int upload_table(Server* sv)
         d.g_spmv = (int)spmv_grid(c, sym, false);
         d.g_vec = (int)vec_grid(d.n);
         d.join = h.join_it;
+        d.form = h.seg.form;
+        d.seg_b = h.seg.g.B;
+        d.seg_r = h.seg.g.R;
+        d.cut = (decltype(d.cut))h.seg.g.cut;
+        d.items = h.seg.items;
         T.pre_spmv[ns] = gs;
         T.pre_vec[ns] = gvv;
-        gs += d.g_spmv;
-        gvv += d.g_vec;
+        T.pre_seg[ns] = gseg;
+        gs += d.seg_b ? 0 : d.g_spmv;
+        gvv += d.seg_b ? 0 : d.g_vec;
+        gseg += h.resident ? 0 : d.seg_b;
+        if (h.resident) {
+            // requests share a launch while its blocks have a compute unit each
+            const int most = beside ? resident_blocks(c->n_cu) * 3 / 4 : resident_blocks(c->n_cu);
+            size_t lds = 0;
+            if (resident_entry(c, h.seg.g, sv->scal + s, &T.cg[ncg], &lds) != INS_OK)
+                return sfail(sv, INS_ERR_HIP, c->err);
+            if (sv->groups.empty() || sv->groups.back().blocks + h.seg.g.B > most)
+                sv->groups.push_back(CgGroup{ncg, 0, 0, 0});
+            CgGroup& g = sv->groups.back();
+            T.cg[ncg].first = g.blocks;
+            g.blocks += h.seg.g.B;
+            g.n++;
+            g.lds = std::max(g.lds, lds);
+            ncg++;
+        }
         ns++;
     }
     T.nslot = ns;
     T.pre_spmv[ns] = gs;
     T.pre_vec[ns] = gvv;
+    T.pre_seg[ns] = gseg;
     sv->grid_spmv = gs;
     sv->grid_vec = gvv;
+    sv->grid_seg = gseg;
     SRV_HIP(sv, hipMemcpyAsync(sv->d_tab + t, &T, sizeof(BatchTab), hipMemcpyHostToDevice,
                                sv->stream));
     SRV_HIP(sv, hipEventRecord(sv->tab_ev[t], sv->stream));
@@ -3689,7 +3981,10 @@ int server_create(Server** out, int device, int max_slots)
                   hipSuccess &&
               hipHostMalloc((void**)&sv->h_tab, Server::NTAB * sizeof(BatchTab), 0) == hipSuccess &&
               hipMalloc((void**)&sv->d_tab, Server::NTAB * sizeof(BatchTab)) == hipSuccess &&
-              hipEventCreateWithFlags(&sv->ev_sync, hipEventDisableTiming) == hipSuccess;
+              hipEventCreateWithFlags(&sv->ev_sync, hipEventDisableTiming) == hipSuccess &&
+              hipStreamCreateWithFlags(&sv->side, hipStreamNonBlocking) == hipSuccess &&
+              hipEventCreateWithFlags(&sv->ev_fork, hipEventDisableTiming) == hipSuccess &&
+              hipEventCreateWithFlags(&sv->ev_join, hipEventDisableTiming) == hipSuccess;
     for (int i = 0; ok && i < Server::NSNAP; i++)
         ok = hipEventCreateWithFlags(&sv->snap_ev[i], hipEventDisableTiming) == hipSuccess;
     for (int i = 0; ok && i < Server::NTAB; i++)
@@ -3711,7 +4006,12 @@ void server_destroy(Server* sv)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : sv->tab_ev)
         if (e) (void)hipEventDestroy(e);
-    if (sv->ev_sync) (void)hipEventDestroy(sv->ev_sync);
+    if (sv->side) {
+        (void)hipStreamSynchronize(sv->side);
+        (void)hipStreamDestroy(sv->side);
+    }
+    for (hipEvent_t e : {sv->ev_sync, sv->ev_fork, sv->ev_join})
+        if (e) (void)hipEventDestroy(e);
     if (sv->scal) (void)hipFree(sv->scal);
     if (sv->d_tab) (void)hipFree(sv->d_tab);
     if (sv->h_snap) (void)hipHostFree(sv->h_snap);
@@ -3746,19 +4046,16 @@ int server_attach(Server* sv, Ctx* c, double rtol, int max_it, int* slot)
     if (c->sell.stale && (st = fill_sell(c)) != INS_OK) return ctx_fail(st);
     c->want_format = INS_FMT_SELL;
     if ((st = ensure_solver_state(c, INS_SOLVE_MIXED)) != INS_OK) return ctx_fail(st);
+    SegSolve seg;
+    if ((st = solve_segments(c, INS_FMT_SELL, true, &seg)) != INS_OK) return ctx_fail(st);
+    bool fits = false;
+    if ((st = resident_fits(c, seg, &fits)) != INS_OK) return ctx_fail(st);
     // the request's own setup (assembly, SELL) precedes its start
     SRV_HIP(sv, hipEventRecord(sv->ev_sync, c->stream));
     SRV_HIP(sv, hipStreamWaitEvent(sv->stream, sv->ev_sync, 0));
-    const int64_t n = c->n_active;
-    const unsigned gv = vec_grid(n);
     if ((st = solve_vectors(c, INS_FMT_SELL, INS_SOLVE_MIXED, sv->stream)) != INS_OK)
         return ctx_fail(st);
-    SRV_HIP(sv, hipMemsetAsync(c->sx64, 0, n * sizeof(double), sv->stream));
-    k_init<float, float><<<gv, VB, 0, sv->stream>>>(n, c->sb, c->x32.p, c->r32.p, c->p32.p,
-                                                    c->sd32, c->partial.p);
-    k_init_fin<<<1, VB, 0, sv->stream>>>(c->partial.p, (int)gv, rtol * rtol, mixed_delta2(),
-                                 sv->scal + s);
-    SRV_HIP(sv, hipGetLastError());
+    INS_TRY(start_request(sv, s, c, rtol));
     SlotH& h = sv->slots[s];
     h = SlotH();
     h.c = c;
@@ -3767,6 +4064,8 @@ int server_attach(Server* sv, Ctx* c, double rtol, int max_it, int* slot)
     h.max_it = max_it;
     h.join_it = sv->it;
     h.join_chunk = sv->chunks;
+    h.seg = seg;
+    h.resident = fits;
     c->have_solution = false;
     sv->nrun++;
     sv->dirty = true;
@@ -3782,13 +4081,35 @@ int server_step(Server* sv, int k, int* n_finished)
     if (sv->nrun > 0) {
         if (sv->dirty) INS_TRY(upload_table(sv));
         const BatchTab* tab = sv->d_tab + sv->tab_cur;
+        for (SlotH& h : sv->slots)
+            if (h.state == INS_SLOT_RUNNING && h.resident &&
+                resident_words(h.c, sv->stream, k) != INS_OK)
+                return sfail(sv, INS_ERR_HIP, h.c->err);
+        const bool fork = !sv->groups.empty() && (sv->grid_spmv || sv->grid_seg);
+        hipStream_t st = fork ? sv->side : sv->stream;
+        if (fork) {
+            SRV_HIP(sv, hipEventRecord(sv->ev_fork, sv->stream));
+            SRV_HIP(sv, hipStreamWaitEvent(st, sv->ev_fork, 0));
+        }
+        if (!sv->groups.empty() &&
+            resident_batch(sv->device, st, tab->cg, sv->groups, k) != INS_OK)
+            return sfail(sv, INS_ERR_HIP, "resident batch launch");
+        if (fork) SRV_HIP(sv, hipEventRecord(sv->ev_join, st));
         for (int i = 0; i < k; i++) {
-            kb_spmv<<<sv->grid_spmv, SB, 0, sv->stream>>>(tab, sv->it);
-            kb_update_xr<<<sv->grid_vec, VB, 0, sv->stream>>>(tab, sv->it);
-            kb_update_p<<<sv->grid_vec, VB, 0, sv->stream>>>(tab, sv->it);
+            if (sv->grid_spmv) {
+                kb_spmv<<<sv->grid_spmv, SB, 0, sv->stream>>>(tab, sv->it);
+                kb_update_xr<<<sv->grid_vec, VB, 0, sv->stream>>>(tab, sv->it);
+                kb_update_p<<<sv->grid_vec, VB, 0, sv->stream>>>(tab, sv->it);
+            }
+            if (sv->grid_seg) {
+                kb_seg_spmv<<<sv->grid_seg, RT, 0, sv->stream>>>(tab, sv->it);
+                kb_seg_xr<<<sv->grid_seg, RT, 0, sv->stream>>>(tab, sv->it);
+                kb_seg_p<<<sv->grid_seg, RT, 0, sv->stream>>>(tab, sv->it);
+            }
             sv->it++;
         }
         SRV_HIP(sv, hipGetLastError());
+        if (fork) SRV_HIP(sv, hipStreamWaitEvent(sv->stream, sv->ev_join, 0));
         const int r = (int)(sv->chunks % Server::NSNAP);
         SRV_HIP(sv, hipMemcpyAsync(sv->h_snap + (size_t)r * sv->max_slots, sv->scal,
                                    sv->max_slots * sizeof(Scal), hipMemcpyDeviceToHost,
@@ -3979,7 +4300,7 @@ int solve_csr_noalloc(int device, void* stream, int64_t n, int64_t nnz, const in
     if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return INS_ERR_HIP;
     // the segments ins_solve would take: its resident kernel has these bits
-    const Seg seg = csr_segments(n, lpr, n_cu);
+    const Seg seg = csr_segments(n, lpr, n_cu, false);
     k_na_dinv<<<grid_for(n, 256), 256, 0, st>>>(n, rp, col, val, dinv);
     k_init<double, double><<<gv, VB, 0, st>>>(n, b, x, r, p, dinv, part);
     k_init_fin<<<1, VB, 0, st>>>(part, (int)gv, rtol * rtol, 0., sc);
@@ -3996,8 +4317,8 @@ int solve_csr_noalloc(int device, void* stream, int64_t n, int64_t nnz, const in
                 else if (lpr == 16) na_seg<16>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
                 else if (lpr == 8) na_seg<8>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
                 else na_seg<4>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
-                k_seg_xr<1, double><<<seg.B, RT, 0, st>>>(n, seg.R, r, q, dinv, part, sc, it);
-                k_seg_p<1, double><<<seg.B, RT, 0, st>>>(n, seg.R, p, r, dinv, part, sc, it, x, x);
+                k_seg_xr<1, double><<<seg.B, RT, 0, st>>>(n, seg, r, q, dinv, part, sc, it);
+                k_seg_p<1, double><<<seg.B, RT, 0, st>>>(n, seg, p, r, dinv, part, sc, it, x, x);
                 continue;
             }
             if (lpr == 32) na_spmv<32>(st, g1, n, rp, col, val, p, q, part, sc, it, R);

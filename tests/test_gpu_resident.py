@@ -66,6 +66,66 @@ def test_csr_resident_equals_segment_kernels(oracle, n, half):
             assert np.linalg.norm(r) <= 1.001e-9 * np.linalg.norm(b) + 1e-13
 
 
+def _sheet_2d(n):
+    """2-D elasticity: node blocks of 2 components"""
+    xyz, conn = P.unit_cube(2, n)
+    return P.linear_elastic_fundsol(xyz, conn, 2)
+
+
+def _half_clamped(n):
+    """neo-Hooke at u = 0 with partly prescribed nodes: full slices"""
+    p = P.neohooke3d(n)
+    p.g[p.meta["right_x"] * 3] = 0.01
+    return p
+
+
+def _poisson_2d(n):
+    p = P.poisson2d(n)
+    p.coef = np.exp(0.5 * P.normal(n, p.conn.shape[0]))[:, None]
+    return p
+
+
+def _q2_2d(n):
+    """2-D degree-2 field with a coefficient per element"""
+    p = P.poisson2d_q2(n)
+    p.coef = np.exp(0.5 * P.normal(n, p.conn.shape[0]))[:, None]
+    return p
+
+
+# storage forms of SELL solves at the edges of their segments: scalar
+# symmetric slices (3-D, 2-D) of one wave's and more slices per wave, node
+# blocks shared out over 8, 4, 3, 2 and 1 waves per slice and several slices
+# per wave, full slices in registers and streamed
+SELL = [(P.diffusion3d, n) for n in (2, 3, 8, 15, 24, 41, 66, 80, 85)]
+SELL += [(_poisson_2d, n) for n in (3, 10, 40, 130, 270, 700)]
+SELL += [(P.elasticity3d, n) for n in (2, 3, 5, 13, 20, 25, 30, 41, 44, 56, 66)]
+SELL += [(_sheet_2d, n) for n in (3, 17, 60, 200, 300, 600)]
+SELL += [(_half_clamped, n) for n in (2, 7, 16, 40, 46)]
+SELL += [(P.diffusion3d_q2, n) for n in (2, 7, 20, 33)] + [(_q2_2d, n) for n in (4, 50)]
+
+
+@pytest.mark.parametrize("make,n", SELL, ids=lambda v: str(getattr(v, "__name__", v)))
+def test_sell_resident_equals_segment_kernels(make, n):
+    prob = make(n)
+    print("case", make.__name__, n, prob.n_active, flush=True)
+    with abi.Context(0) as c:
+        c.load_problem(prob)
+        c.prepare(abi.SOLVE_MIXED, abi.FMT_SELL)
+        c.assemble(abi.FP64)
+        for mode in (abi.SOLVE_MIXED, abi.SOLVE_FP64):
+            got = []
+            for prof in (0, 1, 0):
+                c.set_profiling(prof)
+                # (large systems: enough iterations for a few replacements)
+                it, rel, st = c.solve(mode, abi.FMT_SELL, 1e-8, max_it=400, check=False)
+                assert st in (abi.INS_OK, abi.ERRORS_INV["NOCONV"])
+                got.append((it, rel, st, c.get_solution()))
+            assert got[0][2] == abi.INS_OK or got[0][0] == 400
+            for g in got[1:]:
+                assert g[:3] == got[0][:3]
+                assert np.array_equal(g[3], got[0][3])
+
+
 def test_csr_iteration_limit_and_breakdown():
     rp, ci, val, b = _banded(3000, 4, 5)
     with abi.Context(0) as c:
@@ -96,7 +156,8 @@ out = {}
 with abi.Context(0) as c:
     c.load_problem(P.diffusion3d(20, seed=3))
     c.assemble(abi.FP64)
-    for name, mode, fmt in (("fp64 csr", 0, 0), ("mixed csr", 1, 0)):
+    for name, mode, fmt in (("fp64 csr", 0, 0), ("mixed csr", 1, 0), ("fp64 sell", 0, 1),
+                            ("mixed sell", 1, 1)):
         it, rr, _ = c.solve(mode, fmt, 1e-9)
         out[name] = [it, rr, hashlib.sha256(c.get_solution().tobytes()).hexdigest()]
 print(json.dumps(out), flush=True)
