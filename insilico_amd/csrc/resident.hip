@@ -1536,9 +1536,10 @@ int resident_blocks(int n_cu)
     return n_cu < NXCD ? 0 : std::min(RBMAX, n_cu / NXCD * NXCD);
 }
 
-// Segments of a CSR solve.  R is what eight register passes hold, 8 RT / LPR
-// rows, while that makes no more than the 64 blocks whose sums meet in one
-// stage; beyond them the sums cost the same up to 256 blocks, so all are
+// Segments of a CSR solve.  Up to 64 blocks, whose sums meet in one stage, while
+// eight register passes, 8 RT / LPR rows, hold a segment (1,944 elastic rows:
+// 6.4 us per iteration with 31 blocks, 12.3 with 8 of the largest segments;
+// 15,000 rows of 27: 4.9 and 5.2); beyond them the sums cost the same up to 256 blocks, so all are
 // used (125,000 rows numbered at random, whose windows are gathers of one
 // lane per cycle: C 4.9 us with 123 blocks).  More rows than the registers
 // hold: FP32 rows are streamed, up to CSR_ROWS per block (182,000 rows of 27:
@@ -1551,7 +1552,7 @@ Seg csr_segments(int64_t n, int lpr, int n_cu, bool mixed)
     Seg g;
     if (bmax == 0) return g;
     const int64_t regs = std::max(1, 64 / lpr);
-    int64_t R = regs;
+    int64_t R = std::min<int64_t>(regs, (nsl + 63) / 64);
     if (nsl > 64 * R) R = (nsl + bmax - 1) / bmax;
     if (R > (mixed ? CSR_ROWS / 64 : regs)) return g;
     int64_t B = (nsl + R - 1) / R;

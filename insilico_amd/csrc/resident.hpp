@@ -64,9 +64,8 @@ __device__ inline int opaque_lane()
 // CSR rows: LPR lanes per row, 4 entries per lane in flight (the order of
 // csr_row); p(k) gives the vector value of entry k
 template <int LPR, typename TV, typename TX, class P>
-__device__ inline TX csr_seg_row(int32_t k0, int32_t e, const TV* __restrict__ val, P p)
+__device__ inline TX csr_seg_round(int32_t k0, int32_t e, const TV* __restrict__ val, P p, TX s)
 {
-    TX s = (TX)0;
     for (; k0 < e; k0 += 4 * LPR) {
         TV vv[4];
         TX xx[4];
@@ -79,7 +78,50 @@ __device__ inline TX csr_seg_row(int32_t k0, int32_t e, const TV* __restrict__ v
 #pragma unroll
         for (int j = 0; j < 4; j++) s += (TX)vv[j] * xx[j];
     }
-    return group_sum<LPR>(s);
+    return s;
+}
+template <int LPR, typename TV, typename TX, class P>
+__device__ inline TX csr_seg_row(int32_t k0, int32_t e, const TV* __restrict__ val, P p)
+{
+    return group_sum<LPR>(csr_seg_round<LPR, TV, TX>(k0, e, val, p, (TX)0));
+}
+
+// rows [0, rows) of a segment by THREADS threads, U of a team's rows in flight:
+// f(i, sum) by the first lane of the team
+template <int LPR, int THREADS, int U, typename TV, typename TX, class P, class F>
+__device__ inline void csr_seg_rows(int rows, const int32_t* __restrict__ rp,
+                                    const TV* __restrict__ val, P p, F f)
+{
+    constexpr int T = THREADS / LPR;
+    const int sub = threadIdx.x & (LPR - 1);
+    for (int i0 = threadIdx.x / LPR; i0 < rows; i0 += U * T) {
+        int32_t k0[U], e[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = i0 + u * T;
+            k0[u] = i < rows ? rp[i] + sub : 0;
+            e[u] = i < rows ? rp[i + 1] : 0;
+        }
+        TV vv[U][4];
+        TX xx[U][4];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int32_t k = k0[u] + j * LPR;
+                vv[u][j] = (k < e[u]) ? val[k] : (TV)0;
+                xx[u][j] = (k < e[u]) ? p(k) : (TX)0;
+            }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            TX s = (TX)0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) s += (TX)vv[u][j] * xx[u][j];
+            s = group_sum<LPR>(csr_seg_round<LPR, TV, TX>(k0[u] + 4 * LPR, e[u], val, p, s));
+            const int i = i0 + u * T;
+            if (sub == 0 && i < rows) f(i, s);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -1207,9 +1207,13 @@ __global__ __launch_bounds__(RT) void k_seg_p(int64_t n, Seg g, TX* __restrict__
     update_p_body<TX, TX, SD>(b, n, p, r, dinv, part, g.B, sc, it, x64, x, seg_span(g, b.id));
 }
 
-// K1 on segments of CSR rows (the products and the p.q sums of CsrForm)
+// K1 on segments of CSR rows (the products and the p.q sums of CsrForm).  Twice
+// the threads of CsrForm, and four rows of a team in flight: with a block per
+// compute unit the row products wait for memory.  The sums are those of RT
+// threads, the others add zeros at their end.
+constexpr int SEG_CSR_T = 2 * RT;
 template <int LPR, typename TV, typename TX, typename TVR>
-__global__ __launch_bounds__(RT) void k_seg_csr(int64_t n, int sl_seg,
+__global__ __launch_bounds__(SEG_CSR_T) void k_seg_csr(int64_t n, int sl_seg,
                                                 const int32_t* __restrict__ rp,
                                                 const int32_t* __restrict__ col,
                                                 const TV* __restrict__ val,
@@ -1224,7 +1228,7 @@ __global__ __launch_bounds__(RT) void k_seg_csr(int64_t n, int sl_seg,
     const int rows = (int)(left < 0 ? 0 : (left < most ? left : most));
     if (it == sc->rep_at) {
         double tt = 0., rz = 0.;
-        for (int i = team; i < rows; i += RT / LPR) {
+        for (int i = team; i < rows && threadIdx.x < RT; i += RT / LPR) {
             const int64_t row = row0 + i;
             const double s = csr_row<LPR, TVR, double, double>(row, sub, rp, col, R.val, R.x64);
             if (sub == 0) {
@@ -1241,15 +1245,11 @@ __global__ __launch_bounds__(RT) void k_seg_csr(int64_t n, int sl_seg,
         return;
     }
     if (sc->done || sc->stop) return;
-    for (int i = team; i < rows; i += RT / LPR) {
-        const int32_t e = rp[row0 + i + 1];
-        const TX s = csr_seg_row<LPR, TV, TX>(rp[row0 + i] + sub, e, val,
-                                              [&](int32_t k) { return p[col[k]]; });
-        if (sub == 0) qs[i] = s;
-    }
+    csr_seg_rows<LPR, SEG_CSR_T, 4, TV, TX>(
+        rows, rp + row0, val, [&](int32_t k) { return p[col[k]]; }, [&](int i, TX s) { qs[i] = s; });
     __syncthreads();
     double v[1] = {0.};
-    for (int i = threadIdx.x; i < rows; i += RT) {
+    for (int i = threadIdx.x; i < rows && threadIdx.x < RT; i += RT) {
         const TX qi = qs[i];
         q[row0 + i] = qi;
         v[0] += (double)p[row0 + i] * (double)qi;
@@ -2440,13 +2440,13 @@ int launch_seg_csr_r(Ctx* c, const Seg& g, const TV* val, const TX* p, TX* q, in
     double* part = c->partial.p;
     const int lpr = pick_lpr(c);
     if (lpr == 32)
-        INS_TRY(launch_timed(c, k_seg_csr<32, TV, TX, TVR>, g.B, RT, n, g.R, rp, ci, val, p, q, part, sc, it, R));
+        INS_TRY(launch_timed(c, k_seg_csr<32, TV, TX, TVR>, g.B, SEG_CSR_T, n, g.R, rp, ci, val, p, q, part, sc, it, R));
     else if (lpr == 16)
-        INS_TRY(launch_timed(c, k_seg_csr<16, TV, TX, TVR>, g.B, RT, n, g.R, rp, ci, val, p, q, part, sc, it, R));
+        INS_TRY(launch_timed(c, k_seg_csr<16, TV, TX, TVR>, g.B, SEG_CSR_T, n, g.R, rp, ci, val, p, q, part, sc, it, R));
     else if (lpr == 8)
-        INS_TRY(launch_timed(c, k_seg_csr<8, TV, TX, TVR>, g.B, RT, n, g.R, rp, ci, val, p, q, part, sc, it, R));
+        INS_TRY(launch_timed(c, k_seg_csr<8, TV, TX, TVR>, g.B, SEG_CSR_T, n, g.R, rp, ci, val, p, q, part, sc, it, R));
     else
-        INS_TRY(launch_timed(c, k_seg_csr<4, TV, TX, TVR>, g.B, RT, n, g.R, rp, ci, val, p, q, part, sc, it, R));
+        INS_TRY(launch_timed(c, k_seg_csr<4, TV, TX, TVR>, g.B, SEG_CSR_T, n, g.R, rp, ci, val, p, q, part, sc, it, R));
     INS_HIP_CHECK(c, hipGetLastError());
     return INS_OK;
 }
@@ -4239,7 +4239,7 @@ void na_seg(hipStream_t st, const Seg& g, int64_t n, const int32_t* rp, const in
             const double* val, const double* p, double* q, double* part, const Scal* sc, int it,
             const Rep<double>& R)
 {
-    k_seg_csr<LPR, double, double, double><<<g.B, RT, 0, st>>>(n, g.R, rp, col, val, p, q, part,
+    k_seg_csr<LPR, double, double, double><<<g.B, SEG_CSR_T, 0, st>>>(n, g.R, rp, col, val, p, q, part,
                                                                sc, it, R);
 }
 
