@@ -1790,9 +1790,8 @@ int sell_cuts(Ctx* c, int bmax, Seg* g)
 }  // namespace
 
 // Segments of a SELL solve.  Few blocks meet cheaply (one stage up to 64), so
-// small problems take the largest segments whose entries the registers hold:
-// 16 slices of scalar rows, 4 of node blocks; beyond 64 such segments all
-// compute units are used.
+// small problems take long segments: 16 slices of scalar rows, 4 of node
+// blocks; beyond 64 such segments all compute units are used.
 //
 // Where the registers no longer hold the entries, streaming them through a
 // few waves per compute unit is no better than the three kernels, which sweep
@@ -1800,7 +1799,8 @@ int sell_cuts(Ctx* c, int bmax, Seg* g)
 // resident against three kernels, at the last size held and the next:
 //   scalar rows FP32 (32 slices)   353k rows 13.1 / 16.6, 525k 31.5 / 20.5
 //   scalar rows FP64 (16 slices)   223k rows 10.5 / 23.0, 353k 28.2 / 26.8
-//   node blocks FP32 (5 slices)    67k nodes 9.6 / 23.8,  89k 24.4 / 25.3
+//   node blocks FP32 (7 slices)    89k nodes 11.0 / 25.3; streamed from the
+//     sixth slice on instead of held in LDS the same size took 24.4
 //   full slices FP32 (1280 entries) 223k rows of a degree-2 field 21.8 / 29.0
 // FP64 node blocks gain streamed too (2 slices held: 26k nodes 8.7 / 32.9,
 // streamed: 42k 20.2 / 36.4, 223k 61.6 / 70.2).

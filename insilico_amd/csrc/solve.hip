@@ -2,7 +2,9 @@
 // called by base/solver/Eigen3.hpp:265-275: x0 = 0, z = D^-1 r, stop when
 // |r|^2 < rtol^2 |b|^2 on the recursive residual).
 //
-// Every iteration is three kernels that stream HBM once each:
+// Solves whose matrix fits the registers of the chip run many iterations in
+// one launch (resident.hip).  Beyond that size, every iteration is three
+// kernels that stream HBM once each:
 //   K1  q = A p, per-block partials of p.q
 //   K2  alpha = rho / sum(p.q); x += alpha p; r -= alpha q; partials of r.r, r.D^-1 r
 //   K3  stop test on sum(r.r); beta = sum(r.z) / rho; p = D^-1 r + beta p
@@ -13,6 +15,10 @@
 // an extra launch.  Block 0 records the scalars for the host.  rho is kept in
 // two slots (iteration parity) so that no block reads a slot being written.
 // The host synchronises once per chunk of iterations.
+//
+// The same three kernels exist on the segments of the resident solve (k_seg_*,
+// kb_seg_*): same sums, same bits.  They run profiled solves, solves whose
+// resident launch gave up, and the allocation-free solve.
 //
 // Mixed precision (INS_SOLVE_MIXED): FP32 matrix values and FP32 vectors in
 // K1-K3 with FP32 accumulation in the SpMV and FP64 accumulation of all dot
