@@ -231,17 +231,28 @@ __device__ inline double2 resid_csr(int64_t row0, int rows, const int32_t* rp,
     return v;
 }
 
+template <typename T>
+struct Pair {
+    T a, b;
+};
+
 // The iterations of one block.  F: the matrix form; NR slices per wave, D
 // components per item.  Thread (wave w, lane l) owns items
 // (first + w + RW j) * 64 + l of every component.  r stays in registers; x and
 // the diagonal too where there are few of them, else they are read and
 // written (by their owner only) while a sum travels.
+//
+// F::SHARE_R: the blocks exchange r instead of z and every one scales the r of
+// its window itself, in the expression of the kernels on whole vectors
+// (p = D^-1 r + beta p, D^-1 r unrounded; the reason beside SYM_SUM).  A second,
+// cached load per place of the window.
 template <class F, typename TX>
 __device__ inline void cg_resident(const CgArgs<TX>& a, int launch_iters, int seg, F& f,
                                    TX* __restrict__ win)
 {
     constexpr int NR = F::NR, D = F::D;
     constexpr bool mixed = sizeof(TX) == 4, KEEP = NR * D * sizeof(TX) <= 12;
+    constexpr bool SHARE_R = F::SHARE_R;
     __shared__ double sh[2][RW];
     __shared__ double tot[2][2];
     // scalars that are looked at once an iteration (uniform, but doubles
@@ -331,7 +342,7 @@ __device__ inline void cg_resident(const CgArgs<TX>& a, int launch_iters, int se
                 const TX ri = r[j][c] - al * q[j][c];
                 r[j][c] = ri;
                 const TX zi = d[j][c] * ri;
-                st_agent(&a.z[g], zi);
+                st_agent(&a.z[g], SHARE_R ? ri : zi);
                 v2[0] += (double)ri * (double)ri;
                 v2[1] += (double)ri * (double)zi;
             });
@@ -357,8 +368,12 @@ __device__ inline void cg_resident(const CgArgs<TX>& a, int launch_iters, int se
             if (conv) break;
             const TX be = (TX)(t2[1] / rho);
             rho = t2[1];
-            f.window([&](int64_t g) { return ld_agent(&a.z[g]); },
-                     [&](int i, TX v) { win[i] = v + be * win[i]; });
+            if constexpr (SHARE_R)
+                f.window([&](int64_t g) { return Pair<TX>{ld_agent(&a.z[g]), a.dinv[g]}; },
+                         [&](int i, Pair<TX> v) { win[i] = v.b * v.a + be * win[i]; });
+            else
+                f.window([&](int64_t g) { return ld_agent(&a.z[g]); },
+                         [&](int i, TX v) { win[i] = v + be * win[i]; });
             const bool pause = mixed && rr < s_delta2 * s_rref;
             __syncthreads();
             if (pause) break;
@@ -395,7 +410,7 @@ __device__ inline void cg_resident(const CgArgs<TX>& a, int launch_iters, int se
             items([&](int j, int c, uint32_t g) {
                 r[j][c] = a.r[g];
                 const TX zi = a.dinv[g] * r[j][c];
-                st_agent(&a.z[g], zi);
+                st_agent(&a.z[g], SHARE_R ? r[j][c] : zi);
             });
             stores_done();
             meet_publish<2>(m, v2, sh);
@@ -424,9 +439,14 @@ __device__ inline void cg_resident(const CgArgs<TX>& a, int launch_iters, int se
                 break;
             }
             rho = t2[1];
-            if (restart)
-                f.window([&](int64_t g) { return ld_agent(&a.z[g]); },
-                         [&](int i, TX v) { win[i] = v; });
+            if (restart) {
+                if constexpr (SHARE_R)
+                    f.window([&](int64_t g) { return Pair<TX>{ld_agent(&a.z[g]), a.dinv[g]}; },
+                             [&](int i, Pair<TX> v) { win[i] = v.b * v.a; });
+                else
+                    f.window([&](int64_t g) { return ld_agent(&a.z[g]); },
+                             [&](int i, TX v) { win[i] = v; });
+            }
             __syncthreads();
         }
     }
@@ -473,6 +493,7 @@ __device__ inline void cg_resident(const CgArgs<TX>& a, int launch_iters, int se
 template <int LPR, int NP, typename TV, typename TX>
 struct CsrForm {
     static constexpr int NR = CSR_ROWS / RT, D = 1;
+    static constexpr bool SHARE_R = false;
     const int32_t* rp;
     const int32_t* col;
     const uint16_t* lcol;
@@ -620,9 +641,10 @@ template <int D, typename TX, class L, class O>
 __device__ inline void rel_window(const RelWin& W, int64_t row0, int64_t nn, L load, O op)
 {
     constexpr int U = D == 1 ? 8 : (sizeof(TX) == 4 ? 3 : 2);
+    typedef decltype(load((int64_t)0)) V;   // what is loaded for a place
     const int lane = threadIdx.x & 63;
     for (int c0 = wave_in_block(); c0 < W.npiece; c0 += RW * U) {
-        TX v[U][D];
+        V v[U][D];
         int at[U];
 #pragma unroll
         for (int k = 0; k < U; k++) {
@@ -635,7 +657,7 @@ __device__ inline void rel_window(const RelWin& W, int64_t row0, int64_t nn, L l
                 at[k] = lane < pc.z ? pc.y + lane : -1;
 #pragma unroll
                 for (int d = 0; d < D; d++) {
-                    v[k][d] = 0;
+                    v[k][d] = V{};
                     if (in) v[k][d] = load(d * nn + g);
                 }
             }
@@ -652,6 +674,7 @@ __device__ inline void rel_window(const RelWin& W, int64_t row0, int64_t nn, L l
 template <int NU, int NR_, typename TV, typename TX>
 struct SymForm {
     static constexpr int NR = NR_, D = 1, NT = 2 * NU - 1;
+    static constexpr bool SHARE_R = sizeof(TX) == 4;
     const TV* vals;
     RelWin W;
     int64_t n;
@@ -712,7 +735,14 @@ struct SymForm {
                 for (int t = 0; t < NT; t++) xv[t] = w[li + sh[t]];
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int t = 0; t < NT; t++) s += (TX)rv[j][t] * xv[t];
+                for (int k0 = 0; k0 < NU; k0 += SYM_SUM) {
+#pragma unroll
+                    for (int k = k0; k < k0 + SYM_SUM && k < NU; k++)
+                        s += (TX)rv[j][k ? 2 * k - 1 : 0] * xv[k ? 2 * k - 1 : 0];
+#pragma unroll
+                    for (int k = k0; k < k0 + SYM_SUM && k < NU; k++)
+                        if (k) s += (TX)rv[j][2 * k] * xv[2 * k];
+                }
             }
             q[j][0] = s;
         }
@@ -746,6 +776,7 @@ __global__ __launch_bounds__(RT) void k_cg_sym(CgArgs<TX> a, int iters,
 template <int D_, int NU, int NR_, int PARTS, bool EXT, typename TV, typename TX>
 struct BsymForm {
     static constexpr int NR = NR_, D = D_, NT = 2 * NU - 1, PER = bsym_per(NT, PARTS);
+    static constexpr bool SHARE_R = false;
     // tasks of a wave, and those in registers (all, but for FP32 3 x 3 blocks)
     static constexpr int TW = PARTS == 1 ? 1 : (PARTS == 3 && (EXT || D == 2 || sizeof(TV) == 8) ? 3 : 2);
     static constexpr int TR = EXT ? 2 : TW;
@@ -993,6 +1024,7 @@ constexpr int SELL_SUMS = (SELL_MAXR + TASKS) * 64;
 template <int NR_, int MAXE, typename TV, typename TX>
 struct SellForm {
     static constexpr int NR = NR_, D = 1;
+    static constexpr bool SHARE_R = false;
     SellView S;
     const TV* vals;
     const int32_t* base;

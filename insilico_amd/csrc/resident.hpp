@@ -127,7 +127,16 @@ __device__ inline void csr_seg_rows(int rows, const int32_t* __restrict__ rp,
 // ---------------------------------------------------------------------------
 // Symmetric slices (SymLayout): the 2 NU - 1 entries of a row, or blocks of a
 // node, are numbered t = 0 the diagonal, 2k - 1 the one at offset u_k, 2k its
-// mirror at -u_k, and summed in that order.
+// mirror at -u_k.  Blocks are summed in that order.
+//
+// Scalar rows are summed in the order of the kernels on whole vectors
+// (sym_row_v of solve.hip): SYM_SUM offsets at a time, first their own entries,
+// then the mirrors.  With that, and with p = D^-1 r + beta p rounded as there
+// (update_p_body), a mixed solve takes the same FP32 steps whichever kernels
+// run it.  It matters: by rounding alone 16^3 diffusion solves end after about
+// 103 iterations and 2e-10 off or, one in thirty, after about 91 and 1e-9 to
+// 4e-9 off, both with |b - A x| below the tolerance.
+constexpr int SYM_SUM = 8;
 
 // place of a block's (i, j) entry in the upper triangle of the diagonal block
 template <int D>
@@ -254,6 +263,7 @@ __device__ inline void seg_items(const Span& s, int64_t n, F f)
 
 // forms of the SELL storage that have segments
 enum SegForm { SEG_NONE = 0, SEG_SYM14, SEG_SYM5, SEG_BSYM3, SEG_BSYM2, SEG_SELL };
+__host__ __device__ inline constexpr bool sym_form(int f) { return f == SEG_SYM14 || f == SEG_SYM5; }
 
 // Products of the matrix with x on a segment of a SELL storage, the order of
 // every sum as in the resident kernel's form F: f(place of the item, sum) for
@@ -269,7 +279,7 @@ __device__ inline void seg_products(const Span& sp, int64_t n_, const SellView& 
     auto live = [&](int k) { return k < sl && (s0 + k) * 64 < n; };
     // (the lane is hidden from the optimiser once per slice: it would carry
     // a pointer per entry through the loop over the slices, in scratch)
-    if constexpr (F == SEG_SYM14 || F == SEG_SYM5) {
+    if constexpr (sym_form(F)) {
         constexpr int NU = F == SEG_SYM14 ? 14 : 5;
         int du[NU];
 #pragma unroll
@@ -279,28 +289,32 @@ __device__ inline void seg_products(const Span& sp, int64_t n_, const SellView& 
             const int lane = opaque_lane();
             const int row = (int)(s0 + k) * 64 + lane;
             TX s = (TX)0;
-            // a few offsets at a time (all at once take twice the registers
-            // of the resident kernel's loop)
-            constexpr int G = 5;
+            // own entries and mirrors of SYM_SUM offsets in turn (both at once
+            // take twice the registers of the resident kernel's loop)
 #pragma unroll
-            for (int t0 = 0; t0 < NU; t0 += G) {
-                TV vu[G], vl[G];
-                TX xu[G], xl[G];
+            for (int t0 = 0; t0 < NU; t0 += SYM_SUM) {
+                TV v[SYM_SUM];
+                TX xx[SYM_SUM];
 #pragma unroll
-                for (int g = 0; g < G; g++)
+                for (int g = 0; g < SYM_SUM; g++)
                     if (t0 + g < NU) {
+                        v[g] = sym_seg_own<NU, TV>(vals, s0 + k, lane, t0 + g);
+                        xx[g] = x(min(row + du[t0 + g], n - 1));
+                    }
+#pragma unroll
+                for (int g = 0; g < SYM_SUM; g++)
+                    if (t0 + g < NU) s += (TX)v[g] * xx[g];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int g = 0; g < SYM_SUM; g++)
+                    if (t0 + g > 0 && t0 + g < NU) {
                         const int d = du[t0 + g];
-                        vu[g] = sym_seg_own<NU, TV>(vals, s0 + k, lane, t0 + g);
-                        vl[g] = sym_seg_mirror<NU, TV>(vals, s0 + k, lane, t0 + g, d, edge);
-                        xu[g] = x(min(row + d, n - 1));
-                        xl[g] = x(min(max(row - d, 0), n - 1));
+                        v[g] = sym_seg_mirror<NU, TV>(vals, s0 + k, lane, t0 + g, d, edge);
+                        xx[g] = x(min(max(row - d, 0), n - 1));
                     }
 #pragma unroll
-                for (int g = 0; g < G; g++)
-                    if (t0 + g < NU) {
-                        s += (TX)vu[g] * xu[g];
-                        if (t0 + g > 0) s += (TX)vl[g] * xl[g];
-                    }
+                for (int g = 0; g < SYM_SUM; g++)
+                    if (t0 + g > 0 && t0 + g < NU) s += (TX)v[g] * xx[g];
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (row < n) f(row, s);

@@ -1063,7 +1063,9 @@ __global__ __launch_bounds__(VB) void k_update_xr(int64_t n, TX* __restrict__ x,
 // tolerance, the next iteration is a replacement: every block folds its rows
 // of x32 into x64 here and the leader sets rep_at.  At the replacement
 // iteration K3 restarts the direction if K2 asked for it.
-template <typename TX, typename TD, int SD = 0>
+// ZR (segments): D^-1 r enters p unrounded, as on the whole vectors (the
+// resident forms with SHARE_R); the other forms exchange the rounded z.
+template <typename TX, typename TD, int SD = 0, bool ZR = false>
 __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
                                      const TX* __restrict__ r, const TD* __restrict__ dinv,
                                      const double* part, int g, Scal* sc, int it,
@@ -1135,7 +1137,10 @@ __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
             const TX xi = x[i] + alpha * pi;
             if (fold) x64[i] += (double)xi;
             x[i] = fold ? (TX)0 : xi;
-            if (!conv) {
+            if (conv) return;
+            if constexpr (ZR) {
+                p[i] = dinv[i] * r[i] + beta * pi;
+            } else {
                 const TX zi = dinv[i] * r[i];
                 p[i] = zi + beta * pi;
             }
@@ -1203,14 +1208,14 @@ __global__ __launch_bounds__(RT) void k_seg_xr(int64_t n, Seg g, TX* __restrict_
                                seg_span(g, b.id));
 }
 
-template <int SD, typename TX>
+template <int SD, typename TX, bool ZR = false>
 __global__ __launch_bounds__(RT) void k_seg_p(int64_t n, Seg g, TX* __restrict__ p,
                                               const TX* __restrict__ r,
                                               const TX* __restrict__ dinv, const double* part,
                                               Scal* sc, int it, double* x64, TX* x)
 {
     const Blk b{seg_of_block(blockIdx.x, g.B), g.B};
-    update_p_body<TX, TX, SD>(b, n, p, r, dinv, part, g.B, sc, it, x64, x, seg_span(g, b.id));
+    update_p_body<TX, TX, SD, ZR>(b, n, p, r, dinv, part, g.B, sc, it, x64, x, seg_span(g, b.id));
 }
 
 // K1 on segments of CSR rows (the products and the p.q sums of CsrForm).  Twice
@@ -2559,6 +2564,8 @@ int launch_seg_p(Ctx* c, const SegSolve& s, T* p, const T* r, const T* dinv, T* 
         k_seg_p<3, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     else if (s.D == 2)
         k_seg_p<2, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+    else if (sizeof(T) == 4 && sym_form(s.form))
+        k_seg_p<1, T, true><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     else
         k_seg_p<1, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     INS_HIP_CHECK(c, hipGetLastError());
@@ -3705,13 +3712,13 @@ __global__ __launch_bounds__(RT) void kb_seg_xr(const BatchTab* __restrict__ bt,
     else kb_seg_xr_d<1>(d, b, i);
 }
 
-template <int SD>
+template <int SD, bool ZR>
 __device__ inline void kb_seg_p_d(const SlotDesc& d, Blk b, int i)
 {
-    update_p_body<float, float, SD>(b, d.items, (float*)d.p, (const float*)d.r,
-                                    (const float*)d.dinv, (const double*)d.part, d.seg_b,
-                                    (Scal*)d.sc, i, (double*)d.x64, (float*)d.x,
-                                    seg_span(Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, b.id));
+    update_p_body<float, float, SD, ZR>(b, d.items, (float*)d.p, (const float*)d.r,
+                                        (const float*)d.dinv, (const double*)d.part, d.seg_b,
+                                        (Scal*)d.sc, i, (double*)d.x64, (float*)d.x,
+                                        seg_span(Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, b.id));
 }
 __global__ __launch_bounds__(RT) void kb_seg_p(const BatchTab* __restrict__ bt, int64_t it)
 {
@@ -3719,9 +3726,10 @@ __global__ __launch_bounds__(RT) void kb_seg_p(const BatchTab* __restrict__ bt, 
     const SlotDesc& d = bt->d[s];
     const Blk b{seg_of_block((int)blockIdx.x - bt->pre_seg[s], d.seg_b), d.seg_b};
     const int i = (int)(it - d.join);
-    if (d.form == SEG_BSYM3) kb_seg_p_d<3>(d, b, i);
-    else if (d.form == SEG_BSYM2) kb_seg_p_d<2>(d, b, i);
-    else kb_seg_p_d<1>(d, b, i);
+    if (d.form == SEG_BSYM3) kb_seg_p_d<3, false>(d, b, i);
+    else if (d.form == SEG_BSYM2) kb_seg_p_d<2, false>(d, b, i);
+    else if (sym_form(d.form)) kb_seg_p_d<1, true>(d, b, i);
+    else kb_seg_p_d<1, false>(d, b, i);
 }
 
 }  // namespace

@@ -175,3 +175,37 @@ def test_a_wait_that_is_given_up_falls_back():
         assert r.returncode == 0, r.stderr[-2000:]
         got.append(json.loads(r.stdout.strip().splitlines()[-1]))
     assert got[0] == got[1]
+
+
+SCALAR = r"""
+import hashlib, json
+from insilico_amd import abi, problems as P
+out = {}
+cases = [("3d %d %d" % (n, s), P.diffusion3d(n, seed=s))
+         for n, seeds in ((5, 2), (16, 12), (31, 3), (41, 1), (66, 1)) for s in range(seeds)]
+cases += [("2d %d" % n, P.poisson2d(n)) for n in (7, 40, 130)]
+for name, prob in cases:
+    with abi.Context(0) as c:
+        c.load_problem(prob)
+        c.prepare(abi.SOLVE_MIXED, abi.FMT_SELL)
+        c.assemble(abi.FP64)
+        it, rr, _ = c.solve(abi.SOLVE_MIXED, abi.FMT_SELL, 1e-8)
+        out[name] = [it, hashlib.sha256(c.get_solution().tobytes()).hexdigest()]
+print(json.dumps(out), flush=True)
+"""
+
+
+def test_mixed_scalar_solves_take_the_steps_of_the_plain_kernels():
+    """A mixed solve of scalar symmetric slices rounds every FP32 step as the
+    three kernels on whole vectors do (INS_RESIDENT=0), so it has their
+    iterates: where it stops, and how far from the solution, hangs on rounding.
+    (The FP64 sums are added in another order; no step of these systems feels
+    their last bits.)"""
+    got = []
+    for on in ("1", "0"):
+        env = dict(os.environ, INS_RESIDENT=on)
+        r = subprocess.run([sys.executable, "-c", SCALAR], cwd=ROOT, env=env, capture_output=True,
+                           text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(json.loads(r.stdout.strip().splitlines()[-1]))
+    assert got[0] == got[1]
