@@ -147,8 +147,8 @@ struct WinList {
 
 // Segments and windows of the resident solves (resident.hpp)
 struct Resident {
-    DArr<uint64_t> words;    // device-wide sums and the last epoch used
-    int64_t used = 0;        // epochs used at most
+    DArr<uint64_t> words;    // device-wide sums
+    int64_t used = 0;        // last epoch given to a launch
     WinList csr, sell;       // windows of the CSR rows, of the full slices
     DArr<uint16_t> lcol;     // place of every CSR entry's column in its window
     DArr<int32_t> sell_base; // place of lane 0's column of every slice entry

@@ -63,7 +63,7 @@ struct Meet {
 };
 
 constexpr int MEET_SLOT = (RBMAX + RBMAX / 64) * 4;   // words of one parity
-constexpr int MEET_WORDS = 2 * MEET_SLOT;   // and one more: the last epoch used
+constexpr int MEET_WORDS = 2 * MEET_SLOT;
 
 // publish s as the pair of words at w
 __device__ inline void meet_words(const Meet& m, uint64_t* w, double s)
@@ -264,8 +264,7 @@ __device__ inline void cg_resident(const CgArgs<TX>& a, int launch_iters, int se
     int iters = __builtin_amdgcn_readfirstlane(sc->iters);
     if (iters >= a.limit) return;
     double rho = sc->rho[0];
-    // epochs go on where the last launch on these words ended
-    Meet m{a.words, (uint32_t)a.words[MEET_WORDS] + 1u, a.polls, a.g.B, seg};
+    Meet m{a.words, a.epoch, a.polls, a.g.B, seg};
     const int wave = wave_in_block();
     const int64_t nn = a.n;
     const Span sp = seg_span(a.g, seg);
@@ -462,7 +461,6 @@ __device__ inline void cg_resident(const CgArgs<TX>& a, int launch_iters, int se
     });
     __syncthreads();
     if (seg == 0 && threadIdx.x == 0) {
-        a.words[MEET_WORDS] = m.epoch;
         sc->iters = iters;
         sc->rho[0] = rho;
         sc->rho[1] = rho;
@@ -1242,7 +1240,8 @@ __device__ inline T* in_global(T* const& field)
 enum CgVariant { CG_SYM14_2, CG_SYM14_4, CG_SYM5_2, CG_SYM5_4, CG_BSYM3_8, CG_BSYM3_4, CG_BSYM3_3, CG_BSYM3_X,
                  CG_BSYM2_8, CG_BSYM2_4, CG_BSYM2_3, CG_SELL };
 
-__global__ __launch_bounds__(RT) void k_cg_batch(const CgEntry* __restrict__ tab, int n, int iters)
+__global__ __launch_bounds__(RT) void k_cg_batch(const CgEntry* __restrict__ tab, int n, int iters,
+                                                 CgEpochs first)
 {
     extern __shared__ unsigned char lds[];
     __shared__ int firsts[SELL_MAXR + 1];
@@ -1264,6 +1263,7 @@ __global__ __launch_bounds__(RT) void k_cg_batch(const CgEntry* __restrict__ tab
     a.rep.ratio = e.a.rep.ratio;
     a.sc = in_global(e.a.sc);
     a.words = in_global(e.a.words);
+    a.epoch = first.e[s];
     a.polls = e.a.polls;
     a.limit = e.a.limit;
     const float* vals = in_global(e.vals);
@@ -1528,35 +1528,31 @@ int launch_ordered(Ctx* c, K kernel, int blocks, size_t lds, A... args)
 
 template <typename TX>
 CgArgs<TX> cg_args(Ctx* c, const Seg& g, int64_t n, TX* x, TX* r, TX* p, TX* z, const TX* dinv,
-                   const ResRep& rep, Scal* sc, int limit)
+                   const ResRep& rep, Scal* sc, uint32_t epoch, int limit)
 {
     // bound of a wait: a poll takes about a microsecond
-    static const int polls = env_res("INS_RESIDENT_POLLS", 500000);
-    return CgArgs<TX>{n, g, x, r, p, z, dinv, rep, sc, c->res.words.p, polls, limit};
+    const int polls = env_res("INS_RESIDENT_POLLS", 500000);
+    return CgArgs<TX>{n, g, x, r, p, z, dinv, rep, sc, c->res.words.p, epoch, polls, limit};
 }
 
 }  // namespace
 
-// after a launch that was given up: the epochs of its blocks differ
-int resident_reset(Ctx* c, hipStream_t st)
-{
-    INS_HIP_CHECK(c, hipMemsetAsync(c->res.words.p, 0, (MEET_WORDS + 1) * sizeof(uint64_t), st));
-    c->res.used = 0;
-    return INS_OK;
-}
-
-// The words, with epochs left for `iters` iterations on stream st.  Epochs are
-// 32 bits and start again long before they repeat: a sum would take the words
-// of 2^32 sums ago for its own.
-int resident_words(Ctx* c, hipStream_t st, int iters)
+// The words, and the first epoch of a launch of `iters` iterations on stream st:
+// each launch has a range of epochs of its own, of all it may use, so whatever
+// words a launch left, one that was given up or whose end nobody looked at
+// included, are of no epoch that a later one waits for.  Epochs are 32 bits and
+// start again, on zeroed words, before they would repeat.
+int resident_words(Ctx* c, hipStream_t st, int iters, uint32_t* first)
 {
     Resident& S = c->res;
-    if (!S.words.p) {
-        INS_TRY(ensure(c, S.words, MEET_WORDS + 1));
-        INS_TRY(resident_reset(c, st));
-    }
     const int64_t most = 8 * (int64_t)iters + 64;   // replacements included
-    if (S.used + most > (int64_t)1 << 32) INS_TRY(resident_reset(c, st));
+    const bool fresh = !S.words.p;
+    if (fresh) INS_TRY(ensure(c, S.words, MEET_WORDS));
+    if (fresh || S.used + most > (int64_t)UINT32_MAX) {
+        INS_HIP_CHECK(c, hipMemsetAsync(S.words.p, 0, MEET_WORDS * sizeof(uint64_t), st));
+        S.used = 0;
+    }
+    *first = (uint32_t)S.used + 1u;
     S.used += most;
     return INS_OK;
 }
@@ -1691,8 +1687,10 @@ template <typename T>
 int resident_csr(Ctx* c, const Seg& g, int lpr, const T* val, T* x, T* r, T* p, T* z,
                  const T* dinv, const ResRep& rep, int iters, int limit)
 {
-    INS_TRY(resident_words(c, c->stream, iters));
-    const CgArgs<T> a = cg_args<T>(c, g, c->n_active, x, r, p, z, dinv, rep, c->scal.p, limit);
+    uint32_t epoch;
+    INS_TRY(resident_words(c, c->stream, iters, &epoch));
+    const CgArgs<T> a =
+        cg_args<T>(c, g, c->n_active, x, r, p, z, dinv, rep, c->scal.p, epoch, limit);
     if (lpr == 32) return launch_csr_lpr<32>(c, g, a, iters, val);
     if (lpr == 16) return launch_csr_lpr<16>(c, g, a, iters, val);
     if (lpr == 8) return launch_csr_lpr<8>(c, g, a, iters, val);
@@ -1931,11 +1929,12 @@ template <typename T>
 int resident_sell(Ctx* c, const Seg& g, T* x, T* r, T* p, T* z, const T* dinv,
                   const ResRep& rep, int iters, int limit)
 {
-    INS_TRY(resident_words(c, c->stream, iters));
+    uint32_t epoch;
+    INS_TRY(resident_words(c, c->stream, iters, &epoch));
     Resident& S = c->res;
     const SegForm f = sell_form(c);
     const int64_t items = form_dim(f) > 1 ? c->sell.snodes : c->n_active;
-    const CgArgs<T> a = cg_args<T>(c, g, items, x, r, p, z, dinv, rep, c->scal.p, limit);
+    const CgArgs<T> a = cg_args<T>(c, g, items, x, r, p, z, dinv, rep, c->scal.p, epoch, limit);
     const Sell& L = c->sell;
     const T *sym, *full;
     if constexpr (sizeof(T) == 8) {
@@ -1981,7 +1980,7 @@ int resident_entry(Ctx* c, const Seg& g, Scal* sc, CgEntry* e, size_t* lds)
     rep.ratio = restart_ratio();
     rep.v64 = f == SEG_SELL ? L.v64.p : L.vs64.p;
     e->a = cg_args<float>(c, g, D > 1 ? L.snodes : c->n_active, c->x32.p, c->r32.p, c->p32.p,
-                          c->q32.p, c->sd32, rep, sc, INT32_MAX);
+                          c->q32.p, c->sd32, rep, sc, 0u, INT32_MAX);
     e->vals = f == SEG_SELL ? L.v32.p : L.vs.p;
     e->W = RelWin{S.rel_piece.p, S.rel_n, S.rel_sh.p, L.su.p};
     e->S = SellView{nullptr, L.slice_ptr.p, L.slice_pat.p, L.pat_ptr.p, L.pat_len.p, L.pat_delta.p};
@@ -2004,12 +2003,14 @@ int resident_entry(Ctx* c, const Seg& g, Scal* sc, CgEntry* e, size_t* lds)
 }
 
 int resident_batch(int device, hipStream_t st, const CgEntry* tab, const std::vector<CgGroup>& groups,
-                   int iters)
+                   int iters, const uint32_t* first)
 {
     const hipError_t e = ordered(device, st, [&] {
         for (const CgGroup& g : groups) {
+            CgEpochs ep;
+            std::copy(first + g.first, first + g.first + g.n, ep.e);
             const hipError_t le =
-                launch_alone(st, k_cg_batch, g.blocks, g.lds, tab + g.first, g.n, iters);
+                launch_alone(st, k_cg_batch, g.blocks, g.lds, tab + g.first, g.n, iters, ep);
             if (le != hipSuccess) return le;
         }
         return hipSuccess;

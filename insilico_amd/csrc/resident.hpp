@@ -443,7 +443,8 @@ struct CgArgs {
     const TX* dinv;
     ResRep rep;         // mixed
     Scal* sc;
-    uint64_t* words;    // device-wide sums, then the last epoch used
+    uint64_t* words;    // device-wide sums
+    uint32_t epoch;     // of the launch's first sum (resident_words)
     int polls;          // bound of a wait
     int limit;          // iterations of the solve at most
 };
@@ -467,6 +468,12 @@ struct CgEntry {
     const int32_t *base, *list, *woff, *own0;
 };
 
+constexpr int CG_MAX = 64;   // requests of a batch at most
+// first epochs of the requests of one launch
+struct CgEpochs {
+    uint32_t e[CG_MAX] = {};
+};
+
 // one resident launch of a step: entries cg[first] .. of the table
 struct CgGroup {
     int first = 0, n = 0, blocks = 0;
@@ -475,8 +482,7 @@ struct CgGroup {
 
 // launchers (resident.hip)
 int resident_blocks(int n_cu);
-int resident_reset(Ctx* c, hipStream_t st);
-int resident_words(Ctx* c, hipStream_t st, int iters);
+int resident_words(Ctx* c, hipStream_t st, int iters, uint32_t* first);
 double restart_ratio();   // solve.hip
 Seg csr_segments(int64_t n, int lpr, int n_cu, bool mixed);
 int csr_windows(Ctx* c, const Seg& g, int vec_bytes, bool* fits);
@@ -487,7 +493,7 @@ int resident_csr(Ctx* c, const Seg& g, int lpr, const T* val, T* x, T* r, T* p, 
 // a mixed SELL solve as an entry of a batch, and the LDS it needs
 int resident_entry(Ctx* c, const Seg& g, Scal* sc, CgEntry* e, size_t* lds);
 int resident_batch(int device, hipStream_t st, const CgEntry* tab, const std::vector<CgGroup>& groups,
-                   int iters);
+                   int iters, const uint32_t* first);
 SegForm sell_form(const Ctx* c);
 int sell_segments(Ctx* c, bool mixed, Seg* out);
 int sell_windows(Ctx* c, const Seg& g, int vec_bytes, bool* fits);

@@ -2580,7 +2580,8 @@ int resident_fits(Ctx* c, const SegSolve& s, bool* fits)
     const int vb = s.mixed ? 4 : 8;
     int st = s.format == INS_FMT_CSR ? csr_windows(c, s.g, vb, fits)
                                      : sell_windows(c, s.g, vb, fits);
-    if (st == INS_OK && *fits) st = resident_words(c, c->stream, 0);
+    uint32_t first;
+    if (st == INS_OK && *fits) st = resident_words(c, c->stream, 0, &first);
     if (st == INS_ERR_OOM) *fits = false;
     return st == INS_ERR_OOM ? INS_OK : st;
 }
@@ -3208,10 +3209,7 @@ int solve(Ctx* c, int mode, int format, double rtol, int max_it, int* iters, dou
             gave_up = S.abort != 0;
             finished = !gave_up && (S.done || S.stop || S.iters >= max_it);
         }
-        if (gave_up) {
-            INS_TRY(resident_reset(c, c->stream));
-            INS_TRY(init());
-        }
+        if (gave_up) INS_TRY(init());
     }
     const bool resident = finished;
     if (!finished) {
@@ -3550,7 +3548,7 @@ int solve_direct(Ctx* c, int kind, double* relres)
 // request, on the server stream, between chunks.
 namespace {
 
-constexpr int MAXS = 64;  // requests in one batch
+constexpr int MAXS = CG_MAX;  // requests in one batch
 
 // Device pointers in the table are declared as global memory in the device
 // pass, so the kernels that read them use global and scalar loads (as for
@@ -3840,7 +3838,6 @@ int start_request(Server* sv, int s, Ctx* c, double rtol)
 int restart_on_segments(Server* sv, int s)
 {
     SlotH& h = sv->slots[s];
-    if (resident_reset(h.c, sv->stream) != INS_OK) return sfail(sv, INS_ERR_HIP, h.c->err);
     INS_TRY(start_request(sv, s, h.c, h.rtol));
     h.resident = false;
     h.join_it = sv->it;
@@ -4095,9 +4092,11 @@ int server_step(Server* sv, int k, int* n_finished)
     if (sv->nrun > 0) {
         if (sv->dirty) INS_TRY(upload_table(sv));
         const BatchTab* tab = sv->d_tab + sv->tab_cur;
+        uint32_t first[MAXS];   // in the order of the table's entries
+        int ncg = 0;
         for (SlotH& h : sv->slots)
             if (h.state == INS_SLOT_RUNNING && h.resident &&
-                resident_words(h.c, sv->stream, k) != INS_OK)
+                resident_words(h.c, sv->stream, k, &first[ncg++]) != INS_OK)
                 return sfail(sv, INS_ERR_HIP, h.c->err);
         const bool fork = !sv->groups.empty() && (sv->grid_spmv || sv->grid_seg);
         hipStream_t st = fork ? sv->side : sv->stream;
@@ -4106,7 +4105,7 @@ int server_step(Server* sv, int k, int* n_finished)
             SRV_HIP(sv, hipStreamWaitEvent(st, sv->ev_fork, 0));
         }
         if (!sv->groups.empty() &&
-            resident_batch(sv->device, st, tab->cg, sv->groups, k) != INS_OK)
+            resident_batch(sv->device, st, tab->cg, sv->groups, k, first) != INS_OK)
             return sfail(sv, INS_ERR_HIP, "resident batch launch");
         if (fork) SRV_HIP(sv, hipEventRecord(sv->ev_join, st));
         for (int i = 0; i < k; i++) {

@@ -209,3 +209,36 @@ def test_mixed_scalar_solves_take_the_steps_of_the_plain_kernels():
         assert r.returncode == 0, r.stderr[-2000:]
         got.append(json.loads(r.stdout.strip().splitlines()[-1]))
     assert got[0] == got[1]
+
+
+def _fresh(prob, mode):
+    with abi.Context(0) as c:
+        c.load_problem(prob)
+        c.assemble(abi.FP64)
+        it, rel, _ = c.solve(mode, abi.FMT_SELL, 1e-9)
+        return it, rel, c.get_solution()
+
+
+@pytest.mark.parametrize("make", [P.diffusion3d, P.elasticity3d], ids=["scalar", "blocks"])
+def test_a_cancelled_launch_that_gave_up_leaves_nothing_behind(make, monkeypatch):
+    """A request whose launch gave up leaves before anyone looks at it; the
+    next solves of its context, other systems, must not meet its words"""
+    n = 14
+    first, second, third = (make(n, seed=s) for s in (3, 4, 5))
+    with abi.Context(0) as c, abi.Server(0, 2) as srv:
+        for prob in (second, third):
+            c.load_problem(first)
+            c.assemble(abi.FP64)
+            monkeypatch.setenv("INS_RESIDENT_POLLS", "0")
+            slot = srv.attach(c, 1e-9)
+            srv.step(4)
+            assert srv.poll(slot)[0] == abi.SLOT_RUNNING
+            srv.detach(slot)
+            monkeypatch.delenv("INS_RESIDENT_POLLS")
+            c.load_problem(prob)
+            c.assemble(abi.FP64)
+            for mode in (abi.SOLVE_FP64, abi.SOLVE_MIXED):
+                it, rel, _ = c.solve(mode, abi.FMT_SELL, 1e-9)
+                want = _fresh(prob, mode)
+                assert (it, rel) == want[:2]
+                assert np.array_equal(c.get_solution(), want[2])
