@@ -11,6 +11,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "backoff.hpp"
 #include "insilico_hip.h"
 
 namespace ins {
@@ -149,6 +150,7 @@ struct WinList {
 struct Resident {
     DArr<uint64_t> words;    // device-wide sums
     int64_t used = 0;        // last epoch given to a launch
+    Backoff backoff;         // solves after a launch that gave up
     WinList csr, sell;       // windows of the CSR rows, of the full slices
     DArr<uint16_t> lcol;     // place of every CSR entry's column in its window
     DArr<int32_t> sell_base; // place of lane 0's column of every slice entry

@@ -3199,8 +3199,9 @@ int solve(Ctx* c, int mode, int format, double rtol, int max_it, int* iters, dou
     if (seg.g.B && !c->profiling) {
         bool fits = false;
         INS_TRY(resident_fits(c, seg, &fits));
+        const bool tried = fits && !c->res.backoff.skip();
         bool gave_up = false;
-        while (fits && !finished && !gave_up) {
+        while (tried && !finished && !gave_up) {
             INS_TRY(resident_launch(c, seg, max_it));
             // the last launch as a rule: what follows a solve goes with it
             if (!mixed) INS_TRY(launch_resid(c, format));
@@ -3209,7 +3210,12 @@ int solve(Ctx* c, int mode, int format, double rtol, int max_it, int* iters, dou
             gave_up = S.abort != 0;
             finished = !gave_up && (S.done || S.stop || S.iters >= max_it);
         }
-        if (gave_up) INS_TRY(init());
+        if (gave_up) {
+            c->res.backoff.gave_up();
+            INS_TRY(init());
+        } else if (tried) {
+            c->res.backoff.ended_well();
+        }
     }
     const bool resident = finished;
     if (!finished) {
@@ -3775,6 +3781,7 @@ struct Server {
     // leave most of every compute unit idle, and the chains are independent
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    Backoff backoff;     // requests after a launch that gave up
 };
 
 namespace {
@@ -3848,6 +3855,7 @@ int restart_on_segments(Server* sv, int s)
 
 int process_snapshot(Server* sv, int64_t chunk, const Scal* snap)
 {
+    bool gave_up = false;
     for (int s = 0; s < sv->max_slots; s++) {
         SlotH& h = sv->slots[s];
         if (h.state != INS_SLOT_RUNNING || chunk < h.join_chunk) continue;
@@ -3856,7 +3864,9 @@ int process_snapshot(Server* sv, int64_t chunk, const Scal* snap)
             // a wait of the resident launch was given up: again from the
             // start, by the segment kernels (the same iterates)
             INS_TRY(restart_on_segments(sv, s));
+            gave_up = true;
         } else if (S.fin) {
+            if (h.resident) sv->backoff.ended_well();
             INS_TRY(finish(sv, s, INS_OK, &S));
         } else if (S.breakdown) {
             INS_TRY(finish(sv, s, INS_ERR_BREAKDOWN, &S));
@@ -3872,6 +3882,7 @@ int process_snapshot(Server* sv, int64_t chunk, const Scal* snap)
             INS_TRY(finish(sv, s, INS_ERR_NOCONV, nullptr));
         }
     }
+    if (gave_up) sv->backoff.gave_up();
     return INS_OK;
 }
 
@@ -4076,7 +4087,7 @@ int server_attach(Server* sv, Ctx* c, double rtol, int max_it, int* slot)
     h.join_it = sv->it;
     h.join_chunk = sv->chunks;
     h.seg = seg;
-    h.resident = fits;
+    h.resident = fits && !sv->backoff.skip();
     c->have_solution = false;
     sv->nrun++;
     sv->dirty = true;

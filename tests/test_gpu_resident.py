@@ -242,3 +242,22 @@ def test_a_cancelled_launch_that_gave_up_leaves_nothing_behind(make, monkeypatch
                 want = _fresh(prob, mode)
                 assert (it, rel) == want[:2]
                 assert np.array_equal(c.get_solution(), want[2])
+
+
+def test_solves_after_a_give_up_keep_their_bits(monkeypatch):
+    """the pause after a launch that gave up, and the return to resident ones"""
+    prob = P.diffusion3d(14, seed=6)
+    with abi.Context(0) as c:
+        c.load_problem(prob)
+        c.assemble(abi.FP64)
+        want = None
+        for polls in ["0"] + [None] * 18 + ["0"] + [None] * 2:
+            if polls:
+                monkeypatch.setenv("INS_RESIDENT_POLLS", polls)
+            else:
+                monkeypatch.delenv("INS_RESIDENT_POLLS", raising=False)
+            for mode in (abi.SOLVE_FP64, abi.SOLVE_MIXED):
+                c.solve(mode, abi.FMT_SELL, 1e-9)
+            got = c.get_solution()
+            want = got if want is None else want
+            assert np.array_equal(got, want)
