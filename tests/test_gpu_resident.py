@@ -6,6 +6,7 @@ import json
 import os
 import subprocess
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -261,3 +262,87 @@ def test_solves_after_a_give_up_keep_their_bits(monkeypatch):
             got = c.get_solution()
             want = got if want is None else want
             assert np.array_equal(got, want)
+
+
+# one request of every storage form: scalar slices, node blocks in 3-D and 2-D,
+# full slices (partly prescribed nodes, degree 2), and two too large to be resident
+BATCH = [(P.diffusion3d, 17), (P.elasticity3d, 9), (_sheet_2d, 30), (_half_clamped, 8),
+         (P.diffusion3d_q2, 7), (_poisson_2d, 50), (P.diffusion3d, 75), (P.elasticity3d, 50)]
+
+
+@pytest.mark.parametrize("polls", [None, "0"], ids=["resident", "given up"])
+def test_batch_of_all_forms_has_the_bits_of_its_solves(polls, monkeypatch):
+    """resident launches beside batched kernels on the second stream; with a
+    bound of no polls the resident requests start again on the batched segment
+    kernels"""
+    cs, alone = [], []
+    for make, n in BATCH:
+        c = abi.Context(0)
+        c.load_problem(make(n))
+        c.prepare(abi.SOLVE_MIXED, abi.FMT_SELL)
+        c.assemble(abi.FP64)
+        it, rel, _ = c.solve(abi.SOLVE_MIXED, abi.FMT_SELL, 1e-8)
+        alone.append((it, rel, c.get_solution()))
+        cs.append(c)
+    if polls:
+        monkeypatch.setenv("INS_RESIDENT_POLLS", polls)
+    with abi.Server(0, len(cs)) as srv:
+        for _ in range(2):
+            slots = [srv.attach(c, 1e-8) for c in cs]
+            srv.run_until_done()
+            for (make, n), c, slot, want in zip(BATCH, cs, slots, alone):
+                state, status, it, rel = srv.poll(slot)
+                assert (state, status) == (abi.SLOT_FINISHED, abi.INS_OK)
+                srv.detach(slot)
+                assert it == want[0], (make.__name__, n)
+                assert np.array_equal(c.get_solution(), want[2]), (make.__name__, n)
+    for c in cs:
+        c.close()
+
+
+def test_two_threads_solve_at_once():
+    """launches that wait for one another take turns on the device"""
+    probs = [P.diffusion3d(24, seed=1), P.elasticity3d(12, seed=2), P.diffusion3d(13, seed=3)]
+    want = [_fresh(p, m) for p in probs for m in (abi.SOLVE_FP64, abi.SOLVE_MIXED)]
+    got = [[] for _ in probs]
+
+    def work(k):
+        try:
+            for _ in range(3):
+                got[k].append([_fresh(probs[k], m) for m in (abi.SOLVE_FP64, abi.SOLVE_MIXED)])
+        except Exception as e:   # (the main thread reports it)
+            got[k].append(e)
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(probs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(100)
+    for k in range(len(probs)):
+        assert len(got[k]) == 3
+        for round_ in got[k]:
+            for g, w in zip(round_, want[2 * k:2 * k + 2]):
+                assert g[:2] == w[:2] and np.array_equal(g[2], w[2])
+
+
+# (problem, storage form): the residual that the oracle's own FP64 assembly and
+# product give for the solutions of both kinds of kernels
+ORACLE = [(P.diffusion3d, 15), (_poisson_2d, 40), (P.elasticity3d, 9), (_sheet_2d, 17),
+          (_half_clamped, 7), (P.diffusion3d_q2, 6)]
+
+
+@pytest.mark.parametrize("make,n", ORACLE, ids=lambda v: str(getattr(v, "__name__", v)))
+def test_solutions_against_the_oracle(oracle, make, n):
+    prob = make(n)
+    orp, oci, oval, ob, _ = oracle.assemble(prob)
+    with abi.Context(0) as c:
+        c.load_problem(prob)
+        c.prepare(abi.SOLVE_MIXED, abi.FMT_SELL)
+        c.assemble(abi.FP64)
+        for fmt in (abi.FMT_SELL, abi.FMT_CSR):
+            for mode in (abi.SOLVE_MIXED, abi.SOLVE_FP64):
+                for prof in (0, 1):
+                    c.set_profiling(prof)
+                    c.solve(mode, fmt, 1e-8)
+                    r = ob - oracle.spmv(orp, oci, oval, c.get_solution())
+                    # the device's matrix is the oracle's to 1e-12 of its largest entry
+                    assert np.linalg.norm(r) <= 1.001e-8 * np.linalg.norm(ob) + 1e-10
