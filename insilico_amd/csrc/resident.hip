@@ -1293,7 +1293,7 @@ __global__ __launch_bounds__(RT) void k_cg_batch(const CgEntry* __restrict__ tab
 // ---------------------------------------------------------------------------
 // Windows as lists: a bitmap of the columns of the segment's rows in LDS; a
 // column's place is the number of set bits below it.
-constexpr int64_t WIN_MAXN = (LDS_MAX - 4096) / 8 * 32;   // columns a bitmap and its counts hold
+constexpr int64_t WIN_MAXN = LDS_DYN / 8 * 32;   // columns a bitmap and its counts hold
 
 // what marks and places the columns of a segment: CSR rows, or full slices
 struct WinCsr {
@@ -1511,7 +1511,7 @@ hipError_t launch_alone(hipStream_t st, K kernel, int blocks, size_t lds, A... a
     // one block per compute unit: more than half of its LDS
     lds = std::max<size_t>(lds, LDS_MAX / 2 + 1024);
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_DYN);
     if (e != hipSuccess) return e;
     kernel<<<blocks, RT, lds, st>>>(args...);
     return hipGetLastError();
@@ -1602,8 +1602,7 @@ int list_windows(Ctx* c, WinList& L, const Seg& g, W w, P prep)
     INS_TRY(ensure(c, L.wlen, RBMAX + 1));
     INS_HIP_CHECK(c, hipMemsetAsync(L.wlen.p + RBMAX, 0, sizeof(int32_t), c->stream));
     INS_HIP_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_win_count<W>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)(words * 4)));
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, LDS_DYN));
     k_win_count<W><<<g.B, RT, words * 4, c->stream>>>(w, L.wlen.p, L.wlen.p + RBMAX);
     INS_HIP_CHECK(c, hipGetLastError());
     int32_t len[RBMAX + 1], off[RBMAX + 1];
@@ -1624,8 +1623,7 @@ int list_windows(Ctx* c, WinList& L, const Seg& g, W w, P prep)
         INS_HIP_CHECK(c, hipMemcpyAsync(L.woff.p, off, (g.B + 1) * sizeof(int32_t),
                                         hipMemcpyHostToDevice, c->stream));
         INS_HIP_CHECK(c, hipFuncSetAttribute(reinterpret_cast<const void*>(&k_win_fill<W>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)(words * 8)));
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS_DYN));
         k_win_fill<W><<<g.B, RT, words * 8, c->stream>>>(w, L.woff.p, L.list.p, L.own0.p);
         INS_HIP_CHECK(c, hipGetLastError());
         INS_HIP_CHECK(c, hipStreamSynchronize(c->stream));   // off is on this stack
@@ -1642,7 +1640,7 @@ size_t rel_lds(const Ctx* c, int D, int R, int vec_bytes)
            (D > 1 && vec_bytes == 4 ? bsym_ext_lds(D, D == 3 ? 14 : 5, R) : 0);
 }
 
-bool lds_fits(int64_t bytes) { return bytes <= (int64_t)LDS_MAX - 4096; }
+bool lds_fits(int64_t bytes) { return bytes <= (int64_t)LDS_DYN; }
 }  // namespace
 
 // Windows of the current CSR pattern; fits: whether they fit the LDS beside

@@ -22,6 +22,10 @@ constexpr int TASKS = 16;         // shares of a segment that the waves take in 
 constexpr int CSR_ROWS = 1024;    // rows of a CSR segment at most
 constexpr int RBMAX = 256;        // most segments of a solve
 constexpr int LDS_MAX = 160 * 1024;
+// dynamic LDS of a launch at most, beside the kernels' own few KB.  A kernel's
+// limit is set to this, never to a launch's own size, which another thread's
+// (on another device) could lower before the launch.
+constexpr int LDS_DYN = LDS_MAX - 4096;
 
 // Decomposition of one solve into segments (B = 0: none): R slices of 64 rows
 // per block, or, where cut is set, slices cut[b] .. cut[b + 1] - 1 (at most R)

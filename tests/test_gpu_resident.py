@@ -39,7 +39,7 @@ def _banded(n, half, seed):
 
 
 # rows about the edges of slices, of segments (1024 rows for short rows, 512,
-# 256) and of what a window's bitmap holds; row lengths for 4, 8 and 16 lanes,
+# 256) and of what all segments hold (256 of 1024 rows); row lengths for 4, 8 and 16 lanes,
 # register passes and streamed rows
 CSR = [(1, 1), (2, 1), (63, 2), (64, 2), (65, 2), (1023, 3), (1024, 3), (1025, 3), (4097, 4),
        (511, 9), (513, 9), (5000, 13), (70001, 13), (140000, 10), (700, 30), (4096, 40),
