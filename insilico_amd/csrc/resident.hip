@@ -1569,11 +1569,31 @@ int resident_blocks(int n_cu)
 // 6.4 us per iteration with 31 blocks, 12.3 with 8 of the largest segments;
 // 15,000 rows of 27: 4.9 and 5.2); beyond them the sums cost the same up to 256 blocks, so all are
 // used (125,000 rows numbered at random, whose windows are gathers of one
-// lane per cycle: C 4.9 us with 123 blocks).  More rows than the registers
-// hold: FP32 rows are streamed, up to CSR_ROWS per block (182,000 rows of 27:
-// 18.2 us per iteration against 21.6 with three kernels), FP64 rows keep the
-// three kernels (223,000 rows of 27: 28.3 against 27.7 us).
-Seg csr_segments(int64_t n, int lpr, int n_cu, bool mixed)
+// lane per cycle: C 4.9 us with 123 blocks).
+//
+// Rows that the registers do not hold (more than 4 LPR entries) are streamed
+// each iteration.  That pays while values and places, 10 or 6 bytes an entry,
+// stay near (the L2s hold 4 MB for 32 compute units): us per iteration, streamed
+// and with the three kernels on whole vectors,
+//   LPR 16, elastic rows of 78, FP64   27 MB 14.1 / 17.9   35 MB 20.5 / 20.5   45 MB 25.8 / 22.9
+//                               FP32   30 MB 17.9 / 21.8   34 MB 26.7 / 23.1   41 MB 33.4 / 26.3
+//   LPR 8, scattered rows of 31, FP64  34 MB 34.2 / 54.2   39 MB 38.1 / 57.3
+//          rows of 26, one of 200, FP64 34 MB 19.1 / 25.3
+// csr_windows looks at the longest row.  FP32 rows of at most 4 LPR entries are
+// streamed up to CSR_ROWS per block (258,000 rows of 27: 26.3 / 27.5).  FP64
+// segments are a matter of n and nnz alone, for the allocation-free solve knows no
+// more and has the same bits: where rows of about equal length are neither held
+// nor near there are none.
+// passes of a block over its rows, and the most that registers hold
+constexpr int CSR_PASSES = 8;
+static int csr_passes(const Seg& g, int lpr) { return (g.R * 64 * lpr + RT - 1) / RT; }
+
+static bool csr_near(int64_t nnz, int lpr, int n_cu, int vec_bytes)
+{
+    return nnz * (vec_bytes + 2) <= (int64_t)n_cu * (lpr >= 16 ? 120 << 10 : 160 << 10);
+}
+
+Seg csr_segments(int64_t n, int64_t nnz, int lpr, int n_cu, bool mixed)
 {
     const int bmax = resident_blocks(n_cu);
     const int64_t nsl = (n + 63) / 64;
@@ -1583,6 +1603,7 @@ Seg csr_segments(int64_t n, int lpr, int n_cu, bool mixed)
     int64_t R = std::min<int64_t>(regs, (nsl + 63) / 64);
     if (nsl > 64 * R) R = (nsl + bmax - 1) / bmax;
     if (R > (mixed ? CSR_ROWS / 64 : regs)) return g;
+    if (!mixed && nnz > 4 * lpr * n && !csr_near(nnz, lpr, n_cu, 8)) return g;
     int64_t B = (nsl + R - 1) / R;
     if (B >= NXCD) B = std::min<int64_t>(bmax, (B + NXCD - 1) / NXCD * NXCD);
     g.R = (int)R;
@@ -1644,8 +1665,8 @@ bool lds_fits(int64_t bytes) { return bytes <= (int64_t)LDS_DYN; }
 }  // namespace
 
 // Windows of the current CSR pattern; fits: whether they fit the LDS beside
-// the block's q
-int csr_windows(Ctx* c, const Seg& g, int vec_bytes, bool* fits)
+// the block's q, and the registers or the caches the rows
+int csr_windows(Ctx* c, const Seg& g, int lpr, int vec_bytes, bool* fits)
 {
     Resident& S = c->res;
     INS_TRY(list_windows(c, S.csr, g,
@@ -1655,7 +1676,8 @@ int csr_windows(Ctx* c, const Seg& g, int vec_bytes, bool* fits)
                              w.lcol = S.lcol.p;
                              return INS_OK;
                          }));
-    *fits = lds_fits(((int64_t)CSR_ROWS + S.csr.wmax) * vec_bytes);
+    *fits = lds_fits(((int64_t)CSR_ROWS + S.csr.wmax) * vec_bytes) &&
+            (S.csr.maxlen <= 4 * lpr || csr_near(c->nnz, lpr, c->n_cu, vec_bytes));
     return INS_OK;
 }
 
@@ -1665,7 +1687,7 @@ int launch_csr_lpr(Ctx* c, const Seg& g, const CgArgs<TX>& a, int iters, const T
 {
     const Resident& S = c->res;
     const size_t lds = (size_t)(CSR_ROWS + S.csr.wmax) * sizeof(TX);
-    const int passes = (g.R * 64 * LPR + RT - 1) / RT;
+    const int passes = csr_passes(g, LPR);
     const bool regs = S.csr.maxlen <= 4 * LPR;
 #define INS_CG_CSR(NP)                                                                       \
     return launch_ordered(c, k_cg_csr<LPR, NP, TV, TX>, g.B, lds, a, iters, (const int32_t*)c->row_ptr.p, \
@@ -1674,7 +1696,7 @@ int launch_csr_lpr(Ctx* c, const Seg& g, const CgArgs<TX>& a, int iters, const T
                           (const int32_t*)S.csr.woff.p, (const int32_t*)S.csr.own0.p)
     if (regs && passes <= 2) INS_CG_CSR(2);
     if (regs && passes <= 4) INS_CG_CSR(4);
-    if (regs && passes <= 8) INS_CG_CSR(8);
+    if (regs && passes <= CSR_PASSES) INS_CG_CSR(CSR_PASSES);
     INS_CG_CSR(0);
 #undef INS_CG_CSR
 }

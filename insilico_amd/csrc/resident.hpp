@@ -488,8 +488,8 @@ struct CgGroup {
 int resident_blocks(int n_cu);
 int resident_words(Ctx* c, hipStream_t st, int iters, uint32_t* first);
 double restart_ratio();   // solve.hip
-Seg csr_segments(int64_t n, int lpr, int n_cu, bool mixed);
-int csr_windows(Ctx* c, const Seg& g, int vec_bytes, bool* fits);
+Seg csr_segments(int64_t n, int64_t nnz, int lpr, int n_cu, bool mixed);
+int csr_windows(Ctx* c, const Seg& g, int lpr, int vec_bytes, bool* fits);
 template <typename T>
 int resident_csr(Ctx* c, const Seg& g, int lpr, const T* val, T* x, T* r, T* p, T* z,
                  const T* dinv, const ResRep& rep, int iters, int limit);

@@ -2492,7 +2492,7 @@ int solve_segments(Ctx* c, int format, bool mixed, SegSolve* s)
     s->mixed = mixed;
     s->items = c->n_active;
     if (format == INS_FMT_CSR) {
-        s->g = csr_segments(c->n_active, lpr_for(c->n_active, c->nnz), c->n_cu, mixed);
+        s->g = csr_segments(c->n_active, c->nnz, lpr_for(c->n_active, c->nnz), c->n_cu, mixed);
         return INS_OK;
     }
     const int st = sell_segments(c, mixed, &s->g);
@@ -2572,18 +2572,23 @@ int launch_seg_p(Ctx* c, const SegSolve& s, T* p, const T* r, const T* dinv, T* 
     return INS_OK;
 }
 
-// windows and words of a resident solve; no memory for them: not resident
-int resident_fits(Ctx* c, const SegSolve& s, bool* fits)
+// Windows and words of a resident solve; no memory for them: not resident.  A
+// mixed CSR solve that does not fit leaves its segments too (the kernels on
+// whole vectors are faster there); an FP64 one keeps them, for the bits of the
+// allocation-free solve.
+int resident_fits(Ctx* c, SegSolve& s, bool* fits)
 {
     *fits = false;
     if (!s.g.B) return INS_OK;
+    const bool csr = s.format == INS_FMT_CSR;
     const int vb = s.mixed ? 4 : 8;
-    int st = s.format == INS_FMT_CSR ? csr_windows(c, s.g, vb, fits)
-                                     : sell_windows(c, s.g, vb, fits);
+    int st = csr ? csr_windows(c, s.g, pick_lpr(c), vb, fits) : sell_windows(c, s.g, vb, fits);
     uint32_t first;
     if (st == INS_OK && *fits) st = resident_words(c, c->stream, 0, &first);
-    if (st == INS_ERR_OOM) *fits = false;
-    return st == INS_ERR_OOM ? INS_OK : st;
+    if (st != INS_OK) *fits = false;
+    if (st == INS_ERR_OOM) st = INS_OK;
+    if (csr && s.mixed && !*fits) s.g = Seg{};
+    return st;
 }
 
 // up to RES_ITERS iterations of a resident solve, replacements included
@@ -3196,10 +3201,10 @@ int solve(Ctx* c, int mode, int format, double rtol, int max_it, int* iters, dou
     bool finished = false;
     SegSolve seg;
     INS_TRY(solve_segments(c, format, mixed, &seg));
-    if (seg.g.B && !c->profiling) {
-        bool fits = false;
-        INS_TRY(resident_fits(c, seg, &fits));
-        const bool tried = fits && !c->res.backoff.skip();
+    bool fits = false;
+    INS_TRY(resident_fits(c, seg, &fits));
+    if (fits && !c->profiling) {
+        const bool tried = !c->res.backoff.skip();
         bool gave_up = false;
         while (tried && !finished && !gave_up) {
             INS_TRY(resident_launch(c, seg, max_it));
@@ -4324,7 +4329,7 @@ int solve_csr_noalloc(int device, void* stream, int64_t n, int64_t nnz, const in
     if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return INS_ERR_HIP;
     // the segments ins_solve would take: its resident kernel has these bits
-    const Seg seg = csr_segments(n, lpr, n_cu, false);
+    const Seg seg = csr_segments(n, nnz, lpr, n_cu, false);
     k_na_dinv<<<grid_for(n, 256), 256, 0, st>>>(n, rp, col, val, dinv);
     k_init<double, double><<<gv, VB, 0, st>>>(n, b, x, r, p, dinv, part);
     k_init_fin<<<1, VB, 0, st>>>(part, (int)gv, rtol * rtol, 0., sc);

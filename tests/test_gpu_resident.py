@@ -2,6 +2,7 @@
 meeting through device-wide sums) against the segment kernels (three launches
 per iteration on the same segments): the same bits, iteration counts and
 residuals.  A profiled solve takes the segment kernels."""
+import ctypes as C
 import json
 import os
 import subprocess
@@ -10,8 +11,10 @@ import threading
 
 import numpy as np
 import pytest
+import scipy.sparse
 
 from insilico_amd import abi, problems as P
+import test_zz_no_alloc as noalloc
 
 pytestmark = pytest.mark.gpu
 
@@ -346,3 +349,42 @@ def test_solutions_against_the_oracle(oracle, make, n):
                     r = ob - oracle.spmv(orp, oci, oval, c.get_solution())
                     # the device's matrix is the oracle's to 1e-12 of its largest entry
                     assert np.linalg.norm(r) <= 1.001e-8 * np.linalg.norm(ob) + 1e-10
+
+
+# rows longer than the registers hold, at both sides of what is streamed (FP64
+# up to 39,000 rows of 79, FP32 up to 66,000), and a single long row among short
+# ones; the allocation-free solve has the bits of the FP64 solve on either side
+@pytest.mark.parametrize("n,half,long_row", [(30000, 39, 0), (48000, 39, 0), (72000, 39, 0),
+                                             (60000, 13, 200), (130000, 13, 200)])
+def test_long_rows(oracle, n, half, long_row):
+    rp, ci, val, b = _banded(n, half, n)
+    if long_row:
+        i = np.unique(np.linspace(1, n - 1, long_row).astype(int))
+        a = scipy.sparse.csr_matrix((val, ci, rp), (n, n)) + scipy.sparse.coo_matrix(
+            (np.full(2 * len(i), -1e-3), (np.r_[np.zeros(len(i), int), i],
+                                          np.r_[i, np.zeros(len(i), int)])), (n, n)).tocsr()
+        a.sort_indices()
+        rp, ci, val = a.indptr.astype(np.int32), a.indices.astype(np.int32), a.data
+    with abi.Context(0) as c:
+        c.set_csr(rp, ci, val)
+        c.set_rhs(b)
+        for mode in (abi.SOLVE_MIXED, abi.SOLVE_FP64):
+            got = []
+            for prof in (0, 1):
+                c.set_profiling(prof)
+                it, rel, _ = c.solve(mode, abi.FMT_CSR, 1e-9)
+                got.append((it, rel, c.get_solution()))
+            assert got[0][:2] == got[1][:2]
+            assert np.array_equal(got[0][2], got[1][2])
+            r = b - oracle.spmv(rp, ci, val, got[0][2])
+            assert np.linalg.norm(r) <= 1.001e-9 * np.linalg.norm(b) + 1e-13
+    f, hip = noalloc._noalloc(), noalloc._Hip()
+    try:
+        x = hip.put(np.zeros(n))
+        it, rel = C.c_int(), C.c_double()
+        assert f(0, None, n, len(ci), *(hip.put(v) for v in (rp, ci, val, b)), x, 1e-9, 10000,
+                 C.byref(it), C.byref(rel)) == abi.INS_OK
+        assert (it.value, rel.value) == got[0][:2]
+        assert np.array_equal(hip.get(x, n, np.float64), got[0][2])
+    finally:
+        hip.free()
