@@ -932,12 +932,13 @@ struct V16<double> {
 // x update waits for K3)
 // SD > 0: on the segments of resident.hpp instead (b.id: the segment, seg: its
 // slices, SD components of n items), the items and sums of the resident
-// kernel
+// kernel; pq_per: partials of p.q per segment (one, or k_slice_csr's, one per
+// slice, added up in the order of the segment's waves)
 template <typename TX, typename TD, int SD = 0>
 __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* __restrict__ r,
                                       const TX* __restrict__ p, const TX* __restrict__ q,
                                       const TD* __restrict__ dinv, double* part, int g_pq,
-                                      Scal* sc, int it, Span seg = Span{0, 0})
+                                      Scal* sc, int it, Span seg = Span{0, 0}, int pq_per = 1)
 {
     // everything this kernel waits on before its sweep -- the scalars of
     // the last iterations and this thread's share of K1's p.q partials --
@@ -945,7 +946,17 @@ __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* 
     const int rep_at = sc->rep_at, done = sc->done, stop = sc->stop;
     const double rho_it = sc->rho[it & 1];
     double tpq[1];
-    {
+    if (SD > 0 && pq_per > 1) {
+        tpq[0] = 0.;
+        for (int i = threadIdx.x; i < g_pq; i += blockDim.x) {
+            double w[RW], s = 0.;
+#pragma unroll
+            for (int k = 0; k < RW; k++) w[k] = k < pq_per ? part[P_PQ * MAXG + i * pq_per + k] : 0.;
+#pragma unroll
+            for (int k = 0; k < RW; k++) s += w[k];
+            tpq[0] += s;
+        }
+    } else {
         const int slq[1] = {P_PQ};
         totals_share<1>(part, g_pq, slq, tpq);
     }
@@ -1201,11 +1212,11 @@ template <int SD, typename TX>
 __global__ __launch_bounds__(RT) void k_seg_xr(int64_t n, Seg g, TX* __restrict__ r,
                                                const TX* __restrict__ q,
                                                const TX* __restrict__ dinv, double* part, Scal* sc,
-                                               int it)
+                                               int it, int pq_per = 1)
 {
     const Blk b{seg_of_block(blockIdx.x, g.B), g.B};
     update_xr_body<TX, TX, SD>(b, n, nullptr, r, nullptr, q, dinv, part, g.B, sc, it,
-                               seg_span(g, b.id));
+                               seg_span(g, b.id), pq_per);
 }
 
 template <int SD, typename TX, bool ZR = false>
@@ -1218,7 +1229,8 @@ __global__ __launch_bounds__(RT) void k_seg_p(int64_t n, Seg g, TX* __restrict__
     update_p_body<TX, TX, SD, ZR>(b, n, p, r, dinv, part, g.B, sc, it, x64, x, seg_span(g, b.id));
 }
 
-// K1 on segments of CSR rows (the products and the p.q sums of CsrForm).  Twice
+// K1 on segments of CSR rows (the products and the p.q sums of CsrForm), for mixed
+// solves and FP64 segments of more than RW slices (see k_slice_csr).  Twice
 // the threads of CsrForm, and four rows of a team in flight: with a block per
 // compute unit the row products wait for memory.  The sums are those of RT
 // threads, the others add zeros at their end.
@@ -1267,6 +1279,56 @@ __global__ __launch_bounds__(SEG_CSR_T) void k_seg_csr(int64_t n, int sl_seg,
     }
     const int sl[1] = {P_PQ};
     block_partials<1>(v, part, sl, b);
+}
+
+// K1 of an FP64 CSR solve on segments of at most RW slices: a block per slice, a
+// row per team, so that every row is in flight at once; a segment's p.q is that of
+// its slices (waves of the resident kernel) in order, which K2 adds up.  Per
+// launch, a block per segment (k_seg_csr), a block per slice, and the rows of a
+// whole vector (k_spmv_csr): 6,084 elastic rows 7.5, 4.8 and 4.8 us, 15,000 rows of
+// 27 6.1, 3.7 and 4.3 us.
+template <int LPR>
+constexpr int SLICE_T = LPR < 16 ? 64 * LPR : 1024;
+template <int LPR>
+__global__ __launch_bounds__(SLICE_T<LPR>) void k_slice_csr(int64_t n,
+                                                            const int32_t* __restrict__ rp,
+                                                            const int32_t* __restrict__ col,
+                                                            const double* __restrict__ val,
+                                                            const double* __restrict__ p,
+                                                            double* __restrict__ q, double* part,
+                                                            const Scal* sc)
+{
+    __shared__ double qs[64];
+    const int slice = seg_of_block(blockIdx.x, gridDim.x);
+    const int64_t row0 = (int64_t)slice * 64, left = n - row0;
+    const int rows = (int)(left < 0 ? 0 : (left < 64 ? left : 64));
+    if (sc->done || sc->stop) return;
+    const double pi = (int)threadIdx.x < rows ? p[row0 + threadIdx.x] : 0.;
+    csr_seg_rows<LPR, SLICE_T<LPR>, 64 * LPR / SLICE_T<LPR>, double, double>(
+        rows, rp + row0, val, [&](int32_t k) { return p[col[k]]; },
+        [&](int i, double s) { qs[i] = s; });
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        double v = 0.;
+        if ((int)threadIdx.x < rows) {
+            const double qi = qs[threadIdx.x];
+            q[row0 + threadIdx.x] = qi;
+            v += pi * qi;
+        }
+        v = wave_sum(v);
+        if (threadIdx.x == 0) part[P_PQ * MAXG + slice] = v;
+    }
+}
+
+// whether K1 of an FP64 CSR solve takes the segments' slices (it then leaves R
+// partials of p.q per segment)
+bool by_slices(const Seg& g) { return g.R <= RW; }
+
+// Threads of K2 and K3 on segments: the waves without a slice would add zeros to
+// the sums of the block, those without a partial to its totals
+unsigned seg_threads(const Seg& g)
+{
+    return g.R > RW ? RT : 64u * std::min(RW, std::max(g.R, (g.B + 63) / 64));
 }
 
 // K1 on a segment of a SELL storage (at the replacement iteration the FP64
@@ -2462,8 +2524,26 @@ int launch_seg_csr_r(Ctx* c, const Seg& g, const TV* val, const TX* p, TX* q, in
     return INS_OK;
 }
 
+template <int LPR>
+int launch_slice_csr(Ctx* c, const Seg& g)
+{
+    INS_TRY(launch_timed(c, k_slice_csr<LPR>, g.B * g.R, SLICE_T<LPR>, c->n_active,
+                         (const int32_t*)c->row_ptr.p, (const int32_t*)c->col.p,
+                         (const double*)c->val64.p, (const double*)c->p.p, c->q.p, c->partial.p,
+                         (const Scal*)c->scal.p));
+    INS_HIP_CHECK(c, hipGetLastError());
+    return INS_OK;
+}
+
 int launch_seg_csr(Ctx* c, const Seg& g, bool mixed, int it)
 {
+    if (!mixed && by_slices(g)) {
+        const int lpr = pick_lpr(c);
+        if (lpr == 32) return launch_slice_csr<32>(c, g);
+        if (lpr == 16) return launch_slice_csr<16>(c, g);
+        if (lpr == 8) return launch_slice_csr<8>(c, g);
+        return launch_slice_csr<4>(c, g);
+    }
     if (!mixed)
         return launch_seg_csr_r<double, double, double>(c, g, c->val64.p, c->p.p, c->q.p, it,
                                                         c->val64.p);
@@ -2547,12 +2627,14 @@ int launch_seg_spmv(Ctx* c, const SegSolve& s, int it)
 template <typename T>
 int launch_seg_xr(Ctx* c, const SegSolve& s, T* r, const T* q, const T* dinv, int it)
 {
+    const unsigned th = seg_threads(s.g);
+    const int per = s.format == INS_FMT_CSR && !s.mixed && by_slices(s.g) ? s.g.R : 1;
     if (s.D == 3)
-        k_seg_xr<3, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
+        k_seg_xr<3, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
     else if (s.D == 2)
-        k_seg_xr<2, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
+        k_seg_xr<2, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
     else
-        k_seg_xr<1, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
+        k_seg_xr<1, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it, per);
     INS_HIP_CHECK(c, hipGetLastError());
     return INS_OK;
 }
@@ -2560,14 +2642,15 @@ int launch_seg_xr(Ctx* c, const SegSolve& s, T* r, const T* q, const T* dinv, in
 template <typename T>
 int launch_seg_p(Ctx* c, const SegSolve& s, T* p, const T* r, const T* dinv, T* x, int it)
 {
+    const unsigned th = seg_threads(s.g);
     if (s.D == 3)
-        k_seg_p<3, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+        k_seg_p<3, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     else if (s.D == 2)
-        k_seg_p<2, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+        k_seg_p<2, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     else if (sizeof(T) == 4 && sym_form(s.form))
-        k_seg_p<1, T, true><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+        k_seg_p<1, T, true><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     else
-        k_seg_p<1, T><<<s.g.B, RT, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+        k_seg_p<1, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     INS_HIP_CHECK(c, hipGetLastError());
     return INS_OK;
 }
@@ -4273,6 +4356,13 @@ void na_seg(hipStream_t st, const Seg& g, int64_t n, const int32_t* rp, const in
 }
 
 template <int LPR>
+void na_slice(hipStream_t st, const Seg& g, int64_t n, const int32_t* rp, const int32_t* col,
+              const double* val, const double* p, double* q, double* part, const Scal* sc)
+{
+    k_slice_csr<LPR><<<g.B * g.R, SLICE_T<LPR>, 0, st>>>(n, rp, col, val, p, q, part, sc);
+}
+
+template <int LPR>
 void na_resid(hipStream_t st, unsigned g, int64_t n, const int32_t* rp, const int32_t* col,
               const double* val, const double* x, const double* b, double* part)
 {
@@ -4342,12 +4432,18 @@ int solve_csr_noalloc(int device, void* stream, int64_t n, int64_t nnz, const in
         for (int i = 0; i < k; i++) {
             const int it = enq + i;
             if (seg.B) {
-                if (lpr == 32) na_seg<32>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
-                else if (lpr == 16) na_seg<16>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
-                else if (lpr == 8) na_seg<8>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
-                else na_seg<4>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
-                k_seg_xr<1, double><<<seg.B, RT, 0, st>>>(n, seg, r, q, dinv, part, sc, it);
-                k_seg_p<1, double><<<seg.B, RT, 0, st>>>(n, seg, p, r, dinv, part, sc, it, x, x);
+                if (by_slices(seg)) {
+                    if (lpr == 32) na_slice<32>(st, seg, n, rp, col, val, p, q, part, sc);
+                    else if (lpr == 16) na_slice<16>(st, seg, n, rp, col, val, p, q, part, sc);
+                    else if (lpr == 8) na_slice<8>(st, seg, n, rp, col, val, p, q, part, sc);
+                    else na_slice<4>(st, seg, n, rp, col, val, p, q, part, sc);
+                } else {   // (8 lanes and more: segments of at most RW slices)
+                    na_seg<4>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
+                }
+                const unsigned th = seg_threads(seg);
+                k_seg_xr<1, double><<<seg.B, th, 0, st>>>(n, seg, r, q, dinv, part, sc, it,
+                                                          by_slices(seg) ? seg.R : 1);
+                k_seg_p<1, double><<<seg.B, th, 0, st>>>(n, seg, p, r, dinv, part, sc, it, x, x);
                 continue;
             }
             if (lpr == 32) na_spmv<32>(st, g1, n, rp, col, val, p, q, part, sc, it, R);
