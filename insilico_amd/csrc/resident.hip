@@ -211,7 +211,7 @@ __device__ inline double2 resid_sell(Span sp, int64_t n, SellView S,
 {
     double2 v = make_double2(0., 0.);
     seg_products<FORM, TVR, double>(sp, n, S, u, vals, [&](int i) { return rep.x64[i]; }, part,
-                                    [&](int g, double s) { rep.row(g, s, v); });
+                                    wave_in_block(), [&](int g, double s) { rep.row(g, s, v); });
     return v;
 }
 

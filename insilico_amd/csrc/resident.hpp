@@ -251,14 +251,119 @@ __device__ inline int sell_run(const SellView& S, int64_t s0, int64_t s1, int64_
     return (int)((e + 4 * TASKS - 1) / (4 * TASKS)) * 4;
 }
 
-// f(i) for every item of this thread in the span's segment: the items
-// of the resident kernel in its order (component c of item a at c * n + a)
+// The kernels on segments go by units: what one wave of the resident kernel's
+// block owns, slices w, w + RW, .. of a segment, is a wave's work there too.  The
+// U units of a segment that has any (fewer than RW with few slices) are packed into
+// blocks without regard to segments; a wave leaves the sums over its unit, and a
+// segment's sum is that of its units in order, as block_allsum adds the waves of the
+// resident kernel: the same bits.  With U = RW a block is a segment (two units per
+// wave) and leaves its sums itself, which spares the totals most of their loads.
+constexpr int UT = 256;   // threads of a block
+__host__ __device__ inline int seg_units(int R) { return R < RW ? R : RW; }
+__host__ __device__ inline int unit_blocks(int B, int U)
+{
+    const int b = U == RW ? B : (B * U + UT / 64 - 1) / (UT / 64);
+    return b < NXCD ? b : (b + NXCD - 1) / NXCD * NXCD;
+}
+// partials of a segment with U units
+__host__ __device__ inline int unit_per(int U) { return U == RW ? 1 : U; }
+
+struct SegUnit {
+    Span s;
+    int w;       // the wave of the resident kernel
+};
+
+// The calling wave's units in block b of the segments g: w, w + UT / 64, .. below
+// end of segment seg (one call of a body: inlined, which two would not be)
+struct UnitRange {
+    int seg, w, end;
+    bool whole;   // the block is a segment
+};
+__device__ inline UnitRange unit_range(const Seg& g, int U, Blk b)
+{
+    const int wave = wave_in_block(), id = seg_of_block(b.id, b.n);
+    if (U >= RW) return UnitRange{id < g.B ? id : 0, wave, id < g.B ? RW : 0, true};
+    const int u = id * (UT / 64) + wave;
+    if (u >= g.B * U) return UnitRange{0, 0, 0, false};
+    return UnitRange{u / U, u % U, u % U + 1, false};
+}
+
+// body(unit) for the units of block b
+template <class Body>
+__device__ inline void seg_unit_visit(const Seg& g, int U, Blk b, Body body)
+{
+    const UnitRange k = unit_range(g, U, b);
+    const Span s = seg_span(g, k.seg);
+#pragma unroll 1
+    for (int w = k.w; w < k.end; w += UT / 64) body(SegUnit{s, w});
+}
+
+// body(unit, v): the unit's shares v of NV sums; leaves the sums' partials
+template <int NV, class Body>
+__device__ inline void seg_unit_sums(const Seg& g, int U, Blk b, double* part,
+                                     const int (&slot)[NV], Body body)
+{
+    __shared__ double sh[NV][RW];
+    const UnitRange k = unit_range(g, U, b);
+    const Span s = seg_span(g, k.seg);
+#pragma unroll 1
+    for (int w = k.w; w < k.end; w += UT / 64) {
+        double v[NV] = {};
+        body(SegUnit{s, w}, v);
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            v[i] = wave_sum(v[i]);
+            if ((threadIdx.x & 63) == 0) {
+                if (k.whole) sh[i][w] = v[i];
+                else part[slot[i] * MAXG + k.seg * U + w] = v[i];
+            }
+        }
+    }
+    if (!k.whole || k.end == 0) return;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        if ((int)threadIdx.x == i) {
+            double t = 0.;
+#pragma unroll
+            for (int w = 0; w < RW; w++) t += sh[i][w];
+            part[slot[i] * MAXG + k.seg] = t;
+        }
+}
+
+// this thread's share of the totals of B segments (totals_share), each of `per`
+// partials
+template <int NV>
+__device__ inline void unit_totals_share(const double* part, int B, int per,
+                                         const int (&slot)[NV], double (&t)[NV])
+{
+    if (per == 1) return totals_share<NV>(part, B, slot, t);
+#pragma unroll
+    for (int k = 0; k < NV; k++) t[k] = 0.;
+    for (int i = threadIdx.x; i < B; i += blockDim.x) {
+        double v[NV][RW];
+#pragma unroll
+        for (int k = 0; k < NV; k++)
+#pragma unroll
+            for (int w = 0; w < RW; w++)
+                v[k][w] = w < per ? part[slot[k] * MAXG + i * per + w] : 0.;
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            double s = 0.;
+#pragma unroll
+            for (int w = 0; w < RW; w++) s += v[k][w];
+            t[k] += s;
+        }
+    }
+}
+// f(i) for every item of the unit, in the order of the resident kernel
+// (component c of item a at c * n + a)
 template <int D, class F>
-__device__ inline void seg_items(const Span& s, int64_t n, F f)
+__device__ inline void unit_items(const SegUnit& u, int64_t n, F f)
 {
     const int lane = threadIdx.x & 63;
-    for (int k = wave_in_block(); k < s.sl; k += RW) {
-        const int64_t a = (s.s0 + k) * 64 + lane;
+    for (int k = u.w; k < u.s.sl; k += RW) {
+        const int64_t a = (u.s.s0 + k) * 64 + lane;
         if (a < n)
 #pragma unroll
             for (int c = 0; c < D; c++) f(c * n + a);
@@ -271,13 +376,14 @@ __host__ __device__ inline constexpr bool sym_form(int f) { return f == SEG_SYM1
 
 // Products of the matrix with x on a segment of a SELL storage, the order of
 // every sum as in the resident kernel's form F: f(place of the item, sum) for
-// this thread's items; x(i): the vector; part: LDS for the node blocks' part sums
-template <int F, typename TV, typename TX, class X, class Fn>
+// this thread's items; x(i): the vector.  The block's waves together, part: LDS
+// for the node blocks' part sums; or, part null (UNIT), a wave its unit alone,
+// wave: the resident kernel's
+template <int F, typename TV, typename TX, bool UNIT = false, class X, class Fn>
 __device__ inline void seg_products(const Span& sp, int64_t n_, const SellView& S,
                                     const int32_t* __restrict__ u, const TV* __restrict__ vals,
-                                    X x, TX* part, Fn f)
+                                    X x, TX* part, int wave, Fn f)
 {
-    const int wave = wave_in_block();
     const int64_t s0 = sp.s0;
     const int sl = sp.sl, n = (int)n_;
     auto live = [&](int k) { return k < sl && (s0 + k) * 64 < n; };
@@ -350,10 +456,16 @@ __device__ inline void seg_products(const Span& sp, int64_t n_, const SellView& 
                     if (t + g < t0 + per && t + g < NT) bsym_seg_add<D, TV, TX>(b[g], xx[g], out);
             }
         };
-        if (parts == 1) {
+        if (UNIT || parts == 1) {
             for (int k = wave; live(k); k += RW) {
                 TX out[D];
                 sum(k, 0, out);
+                for (int pt = 1; pt < parts; pt++) {
+                    TX o[D];
+                    sum(k, pt * per, o);
+#pragma unroll
+                    for (int c = 0; c < D; c++) out[c] += o[c];
+                }
                 const int a = (int)(s0 + k) * 64 + (int)(threadIdx.x & 63);
                 if (a < n)
 #pragma unroll

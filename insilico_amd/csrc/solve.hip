@@ -530,15 +530,15 @@ __device__ inline void bsym_node(int64_t a, bool live, int lane, int64_t slice, 
 // consecutive nodes) and takes the neighbouring nodes by wave shifts, 3D
 // instead of D * (2 NU - 1) vector loads of p per node.  The blocks of a
 // line (u = c - 1, c, c + 1) are taken together.  Only for slices whose
-// lines stay inside the nodes (the caller checks).
-template <int D, int NU>
-__device__ inline void bsym_lines_node(int64_t a, int lane, int64_t slice, const SymView& Y,
+// lines stay inside the nodes (the caller checks).  added() is called after
+// every block, in the order of their sum.
+template <int D, int NU, class H>
+__device__ inline void bsym_lines_node(int64_t a, int lane, int64_t slice, int64_t nn,
                                        const float* __restrict__ vals,
                                        const float* __restrict__ p, const int (&du)[NU],
-                                       float (&out)[D])
+                                       float (&out)[D], H added)
 {
     constexpr int T = D * (D + 1) / 2, D2 = D * D;
-    const int64_t nn = Y.nn;
     const int64_t ld = 64 * SymLayout{D, NU}.width();
     const float* __restrict__ own = vals + slice * ld + lane;
 #pragma unroll
@@ -563,14 +563,17 @@ __device__ inline void bsym_lines_node(int64_t a, int lane, int64_t slice, const
         for (int i = 0; i < D; i++)
 #pragma unroll
             for (int j = 0; j < D; j++) out[i] += bv[i <= j ? tri_slot<D>(i, j) : tri_slot<D>(j, i)] * x0[j];
+        added();
 #pragma unroll
         for (int i = 0; i < D; i++)
 #pragma unroll
             for (int j = 0; j < D; j++) out[i] += bu[i * D + j] * xu[j];
+        added();
 #pragma unroll
         for (int i = 0; i < D; i++)
 #pragma unroll
             for (int j = 0; j < D; j++) out[i] += bl[j * D + i] * xl[j];
+        added();
     }
     // lines m: blocks k = 2 + 3m, 3 + 3m, 4 + 3m (u = c - 1, c, c + 1)
 #pragma unroll 1
@@ -602,10 +605,12 @@ __device__ inline void bsym_lines_node(int64_t a, int lane, int64_t slice, const
             for (int i = 0; i < D; i++)
 #pragma unroll
                 for (int j = 0; j < D; j++) out[i] += bu[t][i * D + j] * xu[t][j];
+            added();
 #pragma unroll
             for (int i = 0; i < D; i++)
 #pragma unroll
                 for (int j = 0; j < D; j++) out[i] += bl[t][j * D + i] * xl[t][j];
+            added();
         }
     }
 }
@@ -642,8 +647,8 @@ __device__ inline double bsym_sweep(Blk b, const SymView& Y, const TX* __restric
         if constexpr (sizeof(TV) == 4 && sizeof(TX) == 4 && sizeof(TA) == 4) {
             if (lines && slice >= s_lo && slice <= s_hi) {
                 float o[D];
-                bsym_lines_node<D, NUL>(a, lane, slice, Y, (const float*)vals, (const float*)p,
-                                        du, o);
+                bsym_lines_node<D, NUL>(a, lane, slice, nn, (const float*)vals, (const float*)p,
+                                        du, o, [] {});
 #pragma unroll
                 for (int i = 0; i < D; i++) {
                     const float qs = o[i];
@@ -930,15 +935,14 @@ struct V16<double> {
 
 // K2: alpha from the p.q partials; r -= alpha q; r.r, r.z partials (the
 // x update waits for K3)
-// SD > 0: on the segments of resident.hpp instead (b.id: the segment, seg: its
-// slices, SD components of n items), the items and sums of the resident
-// kernel; pq_per: partials of p.q per segment (one, or k_slice_csr's, one per
-// slice, added up in the order of the segment's waves)
+// SD > 0: on the units of segments instead (resident.hpp; SD components of n
+// items, g_pq segments with per_pq partials of p.q each), the items and sums of the
+// resident kernel
 template <typename TX, typename TD, int SD = 0>
 __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* __restrict__ r,
                                       const TX* __restrict__ p, const TX* __restrict__ q,
                                       const TD* __restrict__ dinv, double* part, int g_pq,
-                                      Scal* sc, int it, Span seg = Span{0, 0}, int pq_per = 1)
+                                      Scal* sc, int it, Seg seg = Seg{}, int U = 0, int per_pq = 1)
 {
     // everything this kernel waits on before its sweep -- the scalars of
     // the last iterations and this thread's share of K1's p.q partials --
@@ -946,19 +950,10 @@ __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* 
     const int rep_at = sc->rep_at, done = sc->done, stop = sc->stop;
     const double rho_it = sc->rho[it & 1];
     double tpq[1];
-    if (SD > 0 && pq_per > 1) {
-        tpq[0] = 0.;
-        for (int i = threadIdx.x; i < g_pq; i += blockDim.x) {
-            double w[RW], s = 0.;
-#pragma unroll
-            for (int k = 0; k < RW; k++) w[k] = k < pq_per ? part[P_PQ * MAXG + i * pq_per + k] : 0.;
-#pragma unroll
-            for (int k = 0; k < RW; k++) s += w[k];
-            tpq[0] += s;
-        }
-    } else {
+    {
         const int slq[1] = {P_PQ};
-        totals_share<1>(part, g_pq, slq, tpq);
+        if constexpr (SD > 0) unit_totals_share<1>(part, g_pq, per_pq, slq, tpq);
+        else totals_share<1>(part, g_pq, slq, tpq);
     }
     if (it == rep_at) {
         // replacement iteration: accept or continue from the true residual
@@ -966,7 +961,12 @@ __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* 
         if (b.id != 0) return;
         double t[2];
         const int sl[2] = {P_TT, P_RZ};
-        totals<2>(part, g_pq, sl, t);
+        if constexpr (SD > 0) {
+            unit_totals_share<2>(part, g_pq, per_pq, sl, t);
+            block_allsum<2>(t);
+        } else {
+            totals<2>(part, g_pq, sl, t);
+        }
         if (threadIdx.x == 0) {
             sc->tt = t[0];
             sc->nrep += 1;
@@ -1017,16 +1017,16 @@ __device__ inline void update_xr_body(Blk b, int64_t n, TX* __restrict__ x, TX* 
     const TX alpha = (TX)ad;
     double rr = 0., rz = 0.;
     if constexpr (SD > 0) {
-        seg_items<SD>(seg, n, [&](int64_t i) {
-            const TX ri = r[i] - alpha * q[i];
-            r[i] = ri;
-            const TX zi = dinv[i] * ri;
-            rr += (double)ri * (double)ri;
-            rz += (double)ri * (double)zi;
-        });
-        double v[2] = {rr, rz};
         const int sl[2] = {P_RR, P_RZ};
-        block_partials<2>(v, part, sl, b);
+        seg_unit_sums<2>(seg, U, b, part, sl, [&](const SegUnit& su, double(&v)[2]) {
+            unit_items<SD>(su, n, [&](int64_t i) {
+                const TX ri = r[i] - alpha * q[i];
+                r[i] = ri;
+                const TX zi = dinv[i] * ri;
+                v[0] += (double)ri * (double)ri;
+                v[1] += (double)ri * (double)zi;
+            });
+        });
         return;
     }
     // 16-byte accesses over the full vectors, then the n % W tail
@@ -1081,7 +1081,7 @@ __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
                                      const TX* __restrict__ r, const TD* __restrict__ dinv,
                                      const double* part, int g, Scal* sc, int it,
                                      double* __restrict__ x64, TX* __restrict__ x,
-                                     Span seg = Span{0, 0})
+                                     Seg seg = Seg{}, int U = 0)
 {
     typedef typename V16<TX>::type VT;
     constexpr int W = V16<TX>::W;
@@ -1100,12 +1100,15 @@ __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
     double t[2];
     {
         const int sl[2] = {P_RR, P_RZ};
-        totals_share<2>(part, g, sl, t);
+        if constexpr (SD > 0) unit_totals_share<2>(part, g, unit_per(U), sl, t);
+        else totals_share<2>(part, g, sl, t);
     }
     if (it == rep_at) {
         if (!restart || done) return;
         if constexpr (SD > 0) {
-            seg_items<SD>(seg, n, [&](int64_t i) { p[i] = dinv[i] * r[i]; });
+            seg_unit_visit(seg, U, b, [&](const SegUnit& su) {
+                unit_items<SD>(su, n, [&](int64_t i) { p[i] = dinv[i] * r[i]; });
+            });
             return;
         }
         for (int64_t i = w.first + threadIdx.x; i < w.end; i += w.stride) pv[i] = dv[i] * rv[i];
@@ -1143,18 +1146,20 @@ __device__ inline void update_p_body(Blk b, int64_t n, TX* __restrict__ p,
     if constexpr (SD > 0) {
         const TX beta = conv ? (TX)0 : (TX)(rz / rho);
         const bool fold = mixed && (conv || pause);
-        seg_items<SD>(seg, n, [&](int64_t i) {
-            const TX pi = p[i];
-            const TX xi = x[i] + alpha * pi;
-            if (fold) x64[i] += (double)xi;
-            x[i] = fold ? (TX)0 : xi;
-            if (conv) return;
-            if constexpr (ZR) {
-                p[i] = dinv[i] * r[i] + beta * pi;
-            } else {
-                const TX zi = dinv[i] * r[i];
-                p[i] = zi + beta * pi;
-            }
+        seg_unit_visit(seg, U, b, [&](const SegUnit& su) {
+            unit_items<SD>(su, n, [&](int64_t i) {
+                const TX pi = p[i];
+                const TX xi = x[i] + alpha * pi;
+                if (fold) x64[i] += (double)xi;
+                x[i] = fold ? (TX)0 : xi;
+                if (conv) return;
+                if constexpr (ZR) {
+                    p[i] = dinv[i] * r[i] + beta * pi;
+                } else {
+                    const TX zi = dinv[i] * r[i];
+                    p[i] = zi + beta * pi;
+                }
+            });
         });
         return;
     }
@@ -1207,26 +1212,27 @@ __global__ __launch_bounds__(VB) void k_update_p(int64_t n, TX* __restrict__ p,
     update_p_body<TX, TD>(grid_blk(), n, p, r, dinv, part, g, sc, it, x64, x);
 }
 
-// K2 and K3 on segments
+// K2 and K3 on segments, U units each
 template <int SD, typename TX>
-__global__ __launch_bounds__(RT) void k_seg_xr(int64_t n, Seg g, TX* __restrict__ r,
+__global__ __launch_bounds__(UT) void k_seg_xr(int64_t n, Seg g, int U, int per_pq,
+                                               TX* __restrict__ r,
                                                const TX* __restrict__ q,
                                                const TX* __restrict__ dinv, double* part, Scal* sc,
-                                               int it, int pq_per = 1)
+                                               int it)
 {
-    const Blk b{seg_of_block(blockIdx.x, g.B), g.B};
+    const Blk b = grid_blk();
     update_xr_body<TX, TX, SD>(b, n, nullptr, r, nullptr, q, dinv, part, g.B, sc, it,
-                               seg_span(g, b.id), pq_per);
+                               g, U, per_pq);
 }
 
 template <int SD, typename TX, bool ZR = false>
-__global__ __launch_bounds__(RT) void k_seg_p(int64_t n, Seg g, TX* __restrict__ p,
+__global__ __launch_bounds__(UT) void k_seg_p(int64_t n, Seg g, int U, TX* __restrict__ p,
                                               const TX* __restrict__ r,
                                               const TX* __restrict__ dinv, const double* part,
                                               Scal* sc, int it, double* x64, TX* x)
 {
-    const Blk b{seg_of_block(blockIdx.x, g.B), g.B};
-    update_p_body<TX, TX, SD, ZR>(b, n, p, r, dinv, part, g.B, sc, it, x64, x, seg_span(g, b.id));
+    const Blk b = grid_blk();
+    update_p_body<TX, TX, SD, ZR>(b, n, p, r, dinv, part, g.B, sc, it, x64, x, g, U);
 }
 
 // K1 on segments of CSR rows (the products and the p.q sums of CsrForm), for mixed
@@ -1282,8 +1288,7 @@ __global__ __launch_bounds__(SEG_CSR_T) void k_seg_csr(int64_t n, int sl_seg,
 }
 
 // K1 of an FP64 CSR solve on segments of at most RW slices: a block per slice, a
-// row per team, so that every row is in flight at once; a segment's p.q is that of
-// its slices (waves of the resident kernel) in order, which K2 adds up.  Per
+// row per team, so that every row is in flight at once; a slice is a unit.  Per
 // launch, a block per segment (k_seg_csr), a block per slice, and the rows of a
 // whole vector (k_spmv_csr): 6,084 elastic rows 7.5, 4.8 and 4.8 us, 15,000 rows of
 // 27 6.1, 3.7 and 4.3 us.
@@ -1320,65 +1325,87 @@ __global__ __launch_bounds__(SLICE_T<LPR>) void k_slice_csr(int64_t n,
     }
 }
 
-// whether K1 of an FP64 CSR solve takes the segments' slices (it then leaves R
-// partials of p.q per segment)
+// whether K1 of an FP64 CSR solve takes the segments' slices
 bool by_slices(const Seg& g) { return g.R <= RW; }
 
-// Threads of K2 and K3 on segments: the waves without a slice would add zeros to
-// the sums of the block, those without a partial to its totals
-unsigned seg_threads(const Seg& g)
-{
-    return g.R > RW ? RT : 64u * std::min(RW, std::max(g.R, (g.B + 63) / 64));
-}
-
-// K1 on a segment of a SELL storage (at the replacement iteration the FP64
-// residual)
+// K1 on a unit of a segment of a SELL storage (at the replacement iteration the
+// FP64 residual)
+// lines: the node offsets are stencil lines; the slices whose lines stay inside the
+// nodes then take the line form of the node blocks, in parts
 template <int F, typename TV, typename TX, typename TVR>
-__device__ inline void seg_spmv_body(Blk b, const Span& sp, int64_t n, const SellView& S,
+__device__ inline void seg_spmv_body(const Seg& g, int U, Blk b, int64_t n, const SellView& S,
                                      const int32_t* __restrict__ u, const TV* __restrict__ vals,
                                      const TX* __restrict__ p, TX* __restrict__ q, double* part,
-                                     const Scal* sc, int it, const Rep<TVR>& R, double* lds)
+                                     const Scal* sc, int it, const Rep<TVR>& R, bool lines = false)
 {
     if (it == sc->rep_at) {
-        double v[2] = {0., 0.};
-        seg_products<F, TVR, double>(sp, n, S, u, R.val, [&](int i) { return R.x64[i]; },
-                                     lds, [&](int g, double s) {
-                                         const double ti = R.b[g] - s;
-                                         v[0] += ti * ti;
-                                         const float rf = (float)ti;
-                                         R.r32[g] = rf;
-                                         v[1] += (double)rf * (double)(R.dinv32[g] * rf);
-                                     });
         const int slot[2] = {P_TT, P_RZ};
-        block_partials<2>(v, part, slot, b);
+        seg_unit_sums<2>(g, U, b, part, slot, [&](const SegUnit& su, double(&v)[2]) {
+            seg_products<F, TVR, double, true>(su.s, n, S, u, R.val,
+                                               [&](int i) { return R.x64[i]; }, nullptr, su.w,
+                                               [&](int i, double s) {
+                                                   const double ti = R.b[i] - s;
+                                                   v[0] += ti * ti;
+                                                   const float rf = (float)ti;
+                                                   R.r32[i] = rf;
+                                                   v[1] += (double)rf * (double)(R.dinv32[i] * rf);
+                                               });
+        });
         return;
     }
     if (sc->done || sc->stop) return;
-    double v[1] = {0.};
-    seg_products<F, TV, TX>(sp, n, S, u, vals, [&](int i) { return p[i]; },
-                            reinterpret_cast<TX*>(lds), [&](int g, TX s) {
-                                q[g] = s;
-                                v[0] += (double)p[g] * (double)s;
-                            });
     const int slot[1] = {P_PQ};
-    block_partials<1>(v, part, slot, b);
-}
-
-constexpr int form_parts_lds(int F)
-{
-    return F == SEG_BSYM3 ? BSYM_TASKS * 3 * 64 : (F == SEG_BSYM2 ? BSYM_TASKS * 2 * 64 : 1);
+    seg_unit_sums<1>(g, U, b, part, slot, [&](const SegUnit& su, double(&v)[1]) {
+        if constexpr (sizeof(TV) == 4 && (F == SEG_BSYM3 || F == SEG_BSYM2)) {
+            constexpr int D = F == SEG_BSYM3 ? 3 : 2, NU = F == SEG_BSYM3 ? 14 : 5;
+            int du[NU];
+#pragma unroll
+            for (int k = 0; k < NU; k++) du[k] = __builtin_amdgcn_readfirstlane(u[k]);
+            const int64_t s_lo = 1 + (du[NU - 1] >> 6), s_hi = (n - 1 - du[NU - 1] - 64) / 64;
+            if (lines && su.s.s0 >= s_lo && su.s.s0 + su.s.sl - 1 <= s_hi) {
+                const int lane = threadIdx.x & 63;
+                const int per = bsym_per(2 * NU - 1, bsym_parts(su.s.sl));
+                for (int k = su.w; k < su.s.sl; k += RW) {
+                    const int64_t slice = su.s.s0 + k, a = slice * 64 + lane;
+                    float o[D], tot[D];
+#pragma unroll
+                    for (int c = 0; c < D; c++) tot[c] = 0.f;
+                    int left = per;
+                    bsym_lines_node<D, NU>(a, lane, slice, n, vals, p, du, o, [&] {
+                        if (--left > 0) return;
+                        left = per;
+#pragma unroll
+                        for (int c = 0; c < D; c++) {
+                            tot[c] += o[c];
+                            o[c] = 0.f;
+                        }
+                    });
+#pragma unroll
+                    for (int c = 0; c < D; c++) {
+                        const float s = tot[c] + o[c];
+                        q[c * n + a] = s;
+                        v[0] += (double)p[c * n + a] * (double)s;
+                    }
+                }
+                return;
+            }
+        }
+        seg_products<F, TV, TX, true>(su.s, n, S, u, vals, [&](int i) { return p[i]; }, nullptr,
+                                      su.w, [&](int i, TX s) {
+                                          q[i] = s;
+                                          v[0] += (double)p[i] * (double)s;
+                                      });
+    });
 }
 
 template <int F, typename TV, typename TX, typename TVR>
-__global__ __launch_bounds__(RT) void k_seg_sell(int64_t n, Seg g, SellView S,
+__global__ __launch_bounds__(UT) void k_seg_sell(int64_t n, Seg g, int U, SellView S,
                                                  const int32_t* __restrict__ u,
                                                  const TV* __restrict__ vals,
                                                  const TX* __restrict__ p, TX* __restrict__ q,
                                                  double* part, const Scal* sc, int it, Rep<TVR> R)
 {
-    __shared__ double lds[form_parts_lds(F)];
-    const Blk b{seg_of_block(blockIdx.x, g.B), g.B};
-    seg_spmv_body<F, TV, TX, TVR>(b, seg_span(g, b.id), n, S, u, vals, p, q, part, sc, it, R, lds);
+    seg_spmv_body<F, TV, TX, TVR>(g, U, grid_blk(), n, S, u, vals, p, q, part, sc, it, R);
 }
 
 // start: x = 0, r = b, p = D^-1 b; partials of b.b and r.z
@@ -2564,6 +2591,16 @@ struct SegSolve {
     int D = 1;          // components per item
     int64_t items = 0;
     bool mixed = false;
+    // units of a segment in the kernels on segments
+    int units() const
+    {
+        return format == INS_FMT_CSR && !(by_slices(g) && !mixed) ? RW : seg_units(g.R);
+    }
+    // partials of p.q that their K1 leaves per segment
+    int per_pq() const
+    {
+        return format == INS_FMT_CSR && by_slices(g) && !mixed ? g.R : unit_per(units());
+    }
 };
 
 int solve_segments(Ctx* c, int format, bool mixed, SegSolve* s)
@@ -2590,7 +2627,8 @@ int launch_seg_sell_f(Ctx* c, const SegSolve& s, const TV* val, const TX* p, TX*
 {
     const Rep<TVR> R{rep_val, c->sx64, c->sb, c->r32.p, c->sd32, 0};
     const Scal* sc = c->scal.p;
-    INS_TRY(launch_timed(c, k_seg_sell<F, TV, TX, TVR>, s.g.B, RT, s.items, s.g, sell_view(c),
+    const int U = s.units();
+    INS_TRY(launch_timed(c, k_seg_sell<F, TV, TX, TVR>, unit_blocks(s.g.B, U), UT, s.items, s.g, U, sell_view(c),
                          (const int32_t*)c->sell.su.p, val, p, q, c->partial.p, sc, it, R));
     INS_HIP_CHECK(c, hipGetLastError());
     return INS_OK;
@@ -2627,14 +2665,13 @@ int launch_seg_spmv(Ctx* c, const SegSolve& s, int it)
 template <typename T>
 int launch_seg_xr(Ctx* c, const SegSolve& s, T* r, const T* q, const T* dinv, int it)
 {
-    const unsigned th = seg_threads(s.g);
-    const int per = s.format == INS_FMT_CSR && !s.mixed && by_slices(s.g) ? s.g.R : 1;
+    const int U = s.units(), nb = unit_blocks(s.g.B, U);
     if (s.D == 3)
-        k_seg_xr<3, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
+        k_seg_xr<3, T><<<nb, UT, 0, c->stream>>>(s.items, s.g, U, s.per_pq(), r, q, dinv, c->partial.p, c->scal.p, it);
     else if (s.D == 2)
-        k_seg_xr<2, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it);
+        k_seg_xr<2, T><<<nb, UT, 0, c->stream>>>(s.items, s.g, U, s.per_pq(), r, q, dinv, c->partial.p, c->scal.p, it);
     else
-        k_seg_xr<1, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, r, q, dinv, c->partial.p, c->scal.p, it, per);
+        k_seg_xr<1, T><<<nb, UT, 0, c->stream>>>(s.items, s.g, U, s.per_pq(), r, q, dinv, c->partial.p, c->scal.p, it);
     INS_HIP_CHECK(c, hipGetLastError());
     return INS_OK;
 }
@@ -2642,15 +2679,15 @@ int launch_seg_xr(Ctx* c, const SegSolve& s, T* r, const T* q, const T* dinv, in
 template <typename T>
 int launch_seg_p(Ctx* c, const SegSolve& s, T* p, const T* r, const T* dinv, T* x, int it)
 {
-    const unsigned th = seg_threads(s.g);
+    const int U = s.units(), nb = unit_blocks(s.g.B, U);
     if (s.D == 3)
-        k_seg_p<3, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+        k_seg_p<3, T><<<nb, UT, 0, c->stream>>>(s.items, s.g, U, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     else if (s.D == 2)
-        k_seg_p<2, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+        k_seg_p<2, T><<<nb, UT, 0, c->stream>>>(s.items, s.g, U, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     else if (sizeof(T) == 4 && sym_form(s.form))
-        k_seg_p<1, T, true><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+        k_seg_p<1, T, true><<<nb, UT, 0, c->stream>>>(s.items, s.g, U, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     else
-        k_seg_p<1, T><<<s.g.B, th, 0, c->stream>>>(s.items, s.g, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
+        k_seg_p<1, T><<<nb, UT, 0, c->stream>>>(s.items, s.g, U, p, r, dinv, c->partial.p, c->scal.p, it, c->sx64, x);
     INS_HIP_CHECK(c, hipGetLastError());
     return INS_OK;
 }
@@ -3759,14 +3796,28 @@ __global__ __launch_bounds__(VB) void kb_update_p(const BatchTab* __restrict__ b
 }
 
 // the same three kernels for the requests that are solved on segments
-__global__ __launch_bounds__(RT) void kb_seg_spmv(const BatchTab* __restrict__ bt, int64_t it)
+struct SegBlk {
+    const SlotDesc& d;
+    Blk b;
+    Seg g;
+    int U;
+    int i;   // the request's iteration
+};
+__device__ inline SegBlk seg_blk(const BatchTab* __restrict__ bt, int64_t it)
 {
-    __shared__ double lds[form_parts_lds(SEG_BSYM3)];
     const int s = find_slot(bt->pre_seg, bt->nslot, blockIdx.x);
     const SlotDesc& d = bt->d[s];
+    const Blk b{(int)blockIdx.x - bt->pre_seg[s], bt->pre_seg[s + 1] - bt->pre_seg[s]};
+    return SegBlk{d, b, Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, seg_units(d.seg_r),
+                  (int)(it - d.join)};
+}
+
+__global__ __launch_bounds__(UT) void kb_seg_spmv(const BatchTab* __restrict__ bt, int64_t it)
+{
+    const SegBlk k = seg_blk(bt, it);
+    const SlotDesc& d = k.d;
     const Rep<double> R{(const double*)d.v64, (const double*)d.x64, (const double*)d.b,
                         (float*)d.r, (const float*)d.dinv, 0};
-    const Blk b{seg_of_block((int)blockIdx.x - bt->pre_seg[s], d.seg_b), d.seg_b};
     const SellView S = sell_of(d.S);
     const int32_t* u = (const int32_t*)d.su;
     const float* sym = (const float*)d.vs;
@@ -3774,54 +3825,46 @@ __global__ __launch_bounds__(RT) void kb_seg_spmv(const BatchTab* __restrict__ b
     float* q = (float*)d.q;
     double* part = (double*)d.part;
     const Scal* sc = (const Scal*)d.sc;
-    const int i = (int)(it - d.join);
-    const Span sp = seg_span(Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, b.id);
     switch (d.form) {
-    case SEG_SYM14: seg_spmv_body<SEG_SYM14, float, float, double>(b, sp, d.items, S, u, sym, p, q, part, sc, i, R, lds); break;
-    case SEG_SYM5: seg_spmv_body<SEG_SYM5, float, float, double>(b, sp, d.items, S, u, sym, p, q, part, sc, i, R, lds); break;
-    case SEG_BSYM3: seg_spmv_body<SEG_BSYM3, float, float, double>(b, sp, d.items, S, u, sym, p, q, part, sc, i, R, lds); break;
-    case SEG_BSYM2: seg_spmv_body<SEG_BSYM2, float, float, double>(b, sp, d.items, S, u, sym, p, q, part, sc, i, R, lds); break;
-    default: seg_spmv_body<SEG_SELL, float, float, double>(b, sp, d.items, S, u, (const float*)d.val, p, q, part, sc, i, R, lds); break;
+    case SEG_SYM14: seg_spmv_body<SEG_SYM14, float, float, double>(k.g, k.U, k.b, d.items, S, u, sym, p, q, part, sc, k.i, R); break;
+    case SEG_SYM5: seg_spmv_body<SEG_SYM5, float, float, double>(k.g, k.U, k.b, d.items, S, u, sym, p, q, part, sc, k.i, R); break;
+    case SEG_BSYM3: seg_spmv_body<SEG_BSYM3, float, float, double>(k.g, k.U, k.b, d.items, S, u, sym, p, q, part, sc, k.i, R, d.slines); break;
+    case SEG_BSYM2: seg_spmv_body<SEG_BSYM2, float, float, double>(k.g, k.U, k.b, d.items, S, u, sym, p, q, part, sc, k.i, R, d.slines); break;
+    default: seg_spmv_body<SEG_SELL, float, float, double>(k.g, k.U, k.b, d.items, S, u, (const float*)d.val, p, q, part, sc, k.i, R); break;
     }
 }
 
 template <int SD>
-__device__ inline void kb_seg_xr_d(const SlotDesc& d, Blk b, int i)
+__device__ inline void kb_seg_xr_d(const SegBlk& k)
 {
-    update_xr_body<float, float, SD>(b, d.items, (float*)nullptr, (float*)d.r, nullptr,
+    const SlotDesc& d = k.d;
+    update_xr_body<float, float, SD>(k.b, d.items, (float*)nullptr, (float*)d.r, nullptr,
                                      (const float*)d.q, (const float*)d.dinv, (double*)d.part,
-                                     d.seg_b, (Scal*)d.sc, i,
-                                     seg_span(Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, b.id));
+                                     d.seg_b, (Scal*)d.sc, k.i, k.g, k.U, unit_per(k.U));
 }
-__global__ __launch_bounds__(RT) void kb_seg_xr(const BatchTab* __restrict__ bt, int64_t it)
+__global__ __launch_bounds__(UT) void kb_seg_xr(const BatchTab* __restrict__ bt, int64_t it)
 {
-    const int s = find_slot(bt->pre_seg, bt->nslot, blockIdx.x);
-    const SlotDesc& d = bt->d[s];
-    const Blk b{seg_of_block((int)blockIdx.x - bt->pre_seg[s], d.seg_b), d.seg_b};
-    const int i = (int)(it - d.join);
-    if (d.form == SEG_BSYM3) kb_seg_xr_d<3>(d, b, i);
-    else if (d.form == SEG_BSYM2) kb_seg_xr_d<2>(d, b, i);
-    else kb_seg_xr_d<1>(d, b, i);
+    const SegBlk k = seg_blk(bt, it);
+    if (k.d.form == SEG_BSYM3) kb_seg_xr_d<3>(k);
+    else if (k.d.form == SEG_BSYM2) kb_seg_xr_d<2>(k);
+    else kb_seg_xr_d<1>(k);
 }
 
 template <int SD, bool ZR>
-__device__ inline void kb_seg_p_d(const SlotDesc& d, Blk b, int i)
+__device__ inline void kb_seg_p_d(const SegBlk& k)
 {
-    update_p_body<float, float, SD, ZR>(b, d.items, (float*)d.p, (const float*)d.r,
+    const SlotDesc& d = k.d;
+    update_p_body<float, float, SD, ZR>(k.b, d.items, (float*)d.p, (const float*)d.r,
                                         (const float*)d.dinv, (const double*)d.part, d.seg_b,
-                                        (Scal*)d.sc, i, (double*)d.x64, (float*)d.x,
-                                        seg_span(Seg{d.seg_b, d.seg_r, (const int32_t*)d.cut}, b.id));
+                                        (Scal*)d.sc, k.i, (double*)d.x64, (float*)d.x, k.g, k.U);
 }
-__global__ __launch_bounds__(RT) void kb_seg_p(const BatchTab* __restrict__ bt, int64_t it)
+__global__ __launch_bounds__(UT) void kb_seg_p(const BatchTab* __restrict__ bt, int64_t it)
 {
-    const int s = find_slot(bt->pre_seg, bt->nslot, blockIdx.x);
-    const SlotDesc& d = bt->d[s];
-    const Blk b{seg_of_block((int)blockIdx.x - bt->pre_seg[s], d.seg_b), d.seg_b};
-    const int i = (int)(it - d.join);
-    if (d.form == SEG_BSYM3) kb_seg_p_d<3, false>(d, b, i);
-    else if (d.form == SEG_BSYM2) kb_seg_p_d<2, false>(d, b, i);
-    else if (sym_form(d.form)) kb_seg_p_d<1, true>(d, b, i);
-    else kb_seg_p_d<1, false>(d, b, i);
+    const SegBlk k = seg_blk(bt, it);
+    if (k.d.form == SEG_BSYM3) kb_seg_p_d<3, false>(k);
+    else if (k.d.form == SEG_BSYM2) kb_seg_p_d<2, false>(k);
+    else if (sym_form(k.d.form)) kb_seg_p_d<1, true>(k);
+    else kb_seg_p_d<1, false>(k);
 }
 
 }  // namespace
@@ -3840,6 +3883,7 @@ struct SlotH {
     bool relres_known = false;
     SegSolve seg;   // the segments of its solve (seg.g.B = 0: none)
     bool resident = false;    // it runs in the resident launches
+    int cg = 0;               // its entry there
 };
 
 struct Server {
@@ -3948,9 +3992,10 @@ int process_snapshot(Server* sv, int64_t chunk, const Scal* snap)
         SlotH& h = sv->slots[s];
         if (h.state != INS_SLOT_RUNNING || chunk < h.join_chunk) continue;
         const Scal& S = snap[s];
-        if (S.abort && h.resident) {
-            // a wait of the resident launch was given up: again from the
-            // start, by the segment kernels (the same iterates)
+        if (S.abort) {
+            // a wait of a resident launch was given up (it may have moved to
+            // the segment kernels since): again from the start, by the
+            // segment kernels (the same iterates)
             INS_TRY(restart_on_segments(sv, s));
             gave_up = true;
         } else if (S.fin) {
@@ -3974,6 +4019,67 @@ int process_snapshot(Server* sv, int64_t chunk, const Scal* snap)
     return INS_OK;
 }
 
+// Bytes that an iteration of a served request moves: its FP32 values, seven vectors
+double request_mb(const SlotH& h)
+{
+    const Sell& L = h.c->sell;
+    return 4e-6 * ((double)(h.seg.form == SEG_SELL ? L.nvals : L.nvs) + 7. * h.c->n_active);
+}
+
+// The resident launches of a step: requests share one while every block has a compute
+// unit (first fit, the largest first: eight requests of 16^3 to 44^3 take three
+// launches, 20.1 ms, and took four in the order of their slots, 21.7).  Beside
+// batched kernels a launch leaves them a quarter of the units (a resident block fills
+// its own): a batch of eight with one that is not resident 23.5 ms, 25.3 without.
+//
+// Launches follow one another, while the batched kernels on segments share three
+// launches among all requests, so many middle-sized requests go faster there, and
+// do: microseconds per iteration of the launches and of the segment kernels, fitted
+// to (ms for a batch, resident / segment kernels / batched on whole vectors)
+//   70k elastic rows   3: 13.8/14.8/13.6  4: 18.7/16.6/15.4  6: 27.9/19.8/18.8
+//   114k elastic rows  3: 17.0/20.2/18.5  5: 28.8/25.2/26.7   202k: 4: 30.4/36.0/33.7
+//   89k scalar rows    2: 5.6/5.2/6.0     6: 16.8/10.8/12.4   223k: 4: 18.0/15.8/18.8
+// A request that has moved to the segment kernels stays there.  Both have the same
+// bits, so a running request can move between two steps.
+std::vector<std::vector<int>> pack_requests(Server* sv)
+{
+    bool beside = false, segs = false;
+    std::vector<int> order;
+    for (int s = 0; s < sv->max_slots; s++) {
+        const SlotH& h = sv->slots[s];
+        if (h.state != INS_SLOT_RUNNING) continue;
+        if (h.resident) order.push_back(s);
+        beside |= !h.resident;
+        segs |= !h.resident && h.seg.g.B > 0;
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+        return sv->slots[a].seg.g.B > sv->slots[b].seg.g.B;
+    });
+    std::vector<std::vector<int>> groups;
+    std::vector<int> blocks;
+    double t_res = 0., t_seg = segs ? 0. : 19.;
+    for (int s : order) {
+        const SlotH& h = sv->slots[s];
+        const int B = h.seg.g.B, all = resident_blocks(h.c->n_cu);
+        const int most = beside ? all * 3 / 4 : all;
+        size_t g = 0;
+        while (g < groups.size() && blocks[g] + B > most) g++;
+        if (g == groups.size()) {
+            groups.emplace_back();
+            blocks.push_back(0);
+            t_res += 4.5 + 0.027 * B;
+        }
+        groups[g].push_back(s);
+        blocks[g] += B;
+        t_seg += 0.25 * request_mb(h);
+    }
+    if (groups.size() > 1 && t_seg < t_res) {
+        for (int s : order) sv->slots[s].resident = false;
+        groups.clear();
+    }
+    return groups;
+}
+
 int upload_table(Server* sv)
 {
     const int t = (sv->tab_cur + 1) % Server::NTAB;
@@ -3981,11 +4087,23 @@ int upload_table(Server* sv)
     BatchTab& T = sv->h_tab[t];
     int ns = 0, gs = 0, gvv = 0, gseg = 0, ncg = 0;
     sv->groups.clear();
-    // beside batched kernels a resident launch leaves them a quarter of the
-    // compute units (a resident block fills its own): a batch of eight
-    // requests, one of them not resident, took 23.5 ms, 25.3 without
-    bool beside = false;
-    for (const SlotH& h : sv->slots) beside |= h.state == INS_SLOT_RUNNING && !h.resident;
+    const std::vector<std::vector<int>> packed = pack_requests(sv);
+    for (const std::vector<int>& members : packed) {
+        CgGroup g;
+        g.first = ncg;
+        for (int s : members) {
+            SlotH& h = sv->slots[s];
+            size_t lds = 0;
+            if (resident_entry(h.c, h.seg.g, sv->scal + s, &T.cg[ncg], &lds) != INS_OK)
+                return sfail(sv, INS_ERR_HIP, h.c->err);
+            T.cg[ncg].first = g.blocks;
+            h.cg = ncg++;
+            g.blocks += h.seg.g.B;
+            g.n++;
+            g.lds = std::max(g.lds, lds);
+        }
+        sv->groups.push_back(g);
+    }
     for (int s = 0; s < sv->max_slots; s++) {
         const SlotH& h = sv->slots[s];
         if (h.state != INS_SLOT_RUNNING) continue;
@@ -4032,22 +4150,7 @@ int upload_table(Server* sv)
         T.pre_seg[ns] = gseg;
         gs += d.seg_b ? 0 : d.g_spmv;
         gvv += d.seg_b ? 0 : d.g_vec;
-        gseg += h.resident ? 0 : d.seg_b;
-        if (h.resident) {
-            // requests share a launch while its blocks have a compute unit each
-            const int most = beside ? resident_blocks(c->n_cu) * 3 / 4 : resident_blocks(c->n_cu);
-            size_t lds = 0;
-            if (resident_entry(c, h.seg.g, sv->scal + s, &T.cg[ncg], &lds) != INS_OK)
-                return sfail(sv, INS_ERR_HIP, c->err);
-            if (sv->groups.empty() || sv->groups.back().blocks + h.seg.g.B > most)
-                sv->groups.push_back(CgGroup{ncg, 0, 0, 0});
-            CgGroup& g = sv->groups.back();
-            T.cg[ncg].first = g.blocks;
-            g.blocks += h.seg.g.B;
-            g.n++;
-            g.lds = std::max(g.lds, lds);
-            ncg++;
-        }
+        gseg += h.resident || !d.seg_b ? 0 : unit_blocks(d.seg_b, seg_units(d.seg_r));
         ns++;
     }
     T.nslot = ns;
@@ -4192,34 +4295,37 @@ int server_step(Server* sv, int k, int* n_finished)
         if (sv->dirty) INS_TRY(upload_table(sv));
         const BatchTab* tab = sv->d_tab + sv->tab_cur;
         uint32_t first[MAXS];   // in the order of the table's entries
-        int ncg = 0;
         for (SlotH& h : sv->slots)
             if (h.state == INS_SLOT_RUNNING && h.resident &&
-                resident_words(h.c, sv->stream, k, &first[ncg++]) != INS_OK)
+                resident_words(h.c, sv->stream, k, &first[h.cg]) != INS_OK)
                 return sfail(sv, INS_ERR_HIP, h.c->err);
-        const bool fork = !sv->groups.empty() && (sv->grid_spmv || sv->grid_seg);
+        // what runs on segments goes beside the kernels on whole vectors, or
+        // resident launches beside the kernels on segments
+        const bool resident = !sv->groups.empty(), whole = sv->grid_spmv > 0;
+        const bool segs = sv->grid_seg > 0;
+        const bool fork = whole ? resident || segs : resident && segs;
         hipStream_t st = fork ? sv->side : sv->stream;
+        hipStream_t st_seg = whole ? st : sv->stream;
         if (fork) {
             SRV_HIP(sv, hipEventRecord(sv->ev_fork, sv->stream));
             SRV_HIP(sv, hipStreamWaitEvent(st, sv->ev_fork, 0));
         }
-        if (!sv->groups.empty() &&
-            resident_batch(sv->device, st, tab->cg, sv->groups, k, first) != INS_OK)
+        if (resident && resident_batch(sv->device, st, tab->cg, sv->groups, k, first) != INS_OK)
             return sfail(sv, INS_ERR_HIP, "resident batch launch");
-        if (fork) SRV_HIP(sv, hipEventRecord(sv->ev_join, st));
         for (int i = 0; i < k; i++) {
-            if (sv->grid_spmv) {
+            if (whole) {
                 kb_spmv<<<sv->grid_spmv, SB, 0, sv->stream>>>(tab, sv->it);
                 kb_update_xr<<<sv->grid_vec, VB, 0, sv->stream>>>(tab, sv->it);
                 kb_update_p<<<sv->grid_vec, VB, 0, sv->stream>>>(tab, sv->it);
             }
-            if (sv->grid_seg) {
-                kb_seg_spmv<<<sv->grid_seg, RT, 0, sv->stream>>>(tab, sv->it);
-                kb_seg_xr<<<sv->grid_seg, RT, 0, sv->stream>>>(tab, sv->it);
-                kb_seg_p<<<sv->grid_seg, RT, 0, sv->stream>>>(tab, sv->it);
+            if (segs) {
+                kb_seg_spmv<<<sv->grid_seg, UT, 0, st_seg>>>(tab, sv->it);
+                kb_seg_xr<<<sv->grid_seg, UT, 0, st_seg>>>(tab, sv->it);
+                kb_seg_p<<<sv->grid_seg, UT, 0, st_seg>>>(tab, sv->it);
             }
             sv->it++;
         }
+        if (fork) SRV_HIP(sv, hipEventRecord(sv->ev_join, st));
         SRV_HIP(sv, hipGetLastError());
         if (fork) SRV_HIP(sv, hipStreamWaitEvent(sv->stream, sv->ev_join, 0));
         const int r = (int)(sv->chunks % Server::NSNAP);
@@ -4440,10 +4546,11 @@ int solve_csr_noalloc(int device, void* stream, int64_t n, int64_t nnz, const in
                 } else {   // (8 lanes and more: segments of at most RW slices)
                     na_seg<4>(st, seg, n, rp, col, val, p, q, part, sc, it, R);
                 }
-                const unsigned th = seg_threads(seg);
-                k_seg_xr<1, double><<<seg.B, th, 0, st>>>(n, seg, r, q, dinv, part, sc, it,
-                                                          by_slices(seg) ? seg.R : 1);
-                k_seg_p<1, double><<<seg.B, th, 0, st>>>(n, seg, p, r, dinv, part, sc, it, x, x);
+                const int U = by_slices(seg) ? seg_units(seg.R) : RW;
+                const int nb = unit_blocks(seg.B, U);
+                k_seg_xr<1, double><<<nb, UT, 0, st>>>(n, seg, U, by_slices(seg) ? seg.R : 1, r, q,
+                                                      dinv, part, sc, it);
+                k_seg_p<1, double><<<nb, UT, 0, st>>>(n, seg, U, p, r, dinv, part, sc, it, x, x);
                 continue;
             }
             if (lpr == 32) na_spmv<32>(st, g1, n, rp, col, val, p, q, part, sc, it, R);

@@ -303,6 +303,43 @@ def test_batch_of_all_forms_has_the_bits_of_its_solves(polls, monkeypatch):
         c.close()
 
 
+@pytest.mark.parametrize("make,n,polls", [(P.elasticity3d, 28, None), (P.diffusion3d, 44, None),
+                                          (P.elasticity3d, 28, "0")],
+                         ids=["blocks", "scalar", "given up"])
+def test_running_requests_move_to_the_segment_kernels(make, n, polls, monkeypatch):
+    """two requests run resident for some steps; four more arrive, and the
+    launches of six would take longer than the batched segment kernels: all
+    move there and end with the bits of their solves, also where a launch gave
+    up just before"""
+    cs, alone = [], []
+    for k in range(6):
+        c = abi.Context(0)
+        c.load_problem(make(n, seed=k))
+        c.prepare(abi.SOLVE_MIXED, abi.FMT_SELL)
+        c.assemble(abi.FP64)
+        it, rel, _ = c.solve(abi.SOLVE_MIXED, abi.FMT_SELL, 1e-8)
+        alone.append((it, c.get_solution()))
+        cs.append(c)
+    with abi.Server(0, 6) as srv:
+        slots = [srv.attach(c, 1e-8) for c in cs[:2]]
+        for _ in range(4):
+            srv.step(7)
+        if polls:
+            monkeypatch.setenv("INS_RESIDENT_POLLS", polls)
+            slots += [srv.attach(cs[2], 1e-8)]   # (a new table: the bound goes with it)
+            srv.step(7)
+        slots += [srv.attach(c, 1e-8) for c in cs[len(slots):]]
+        srv.run_until_done()
+        for c, slot, want in zip(cs, slots, alone):
+            state, status, it, _ = srv.poll(slot)
+            assert (state, status) == (abi.SLOT_FINISHED, abi.INS_OK)
+            srv.detach(slot)
+            assert it == want[0]
+            assert np.array_equal(c.get_solution(), want[1])
+    for c in cs:
+        c.close()
+
+
 def test_two_threads_solve_at_once():
     """launches that wait for one another take turns on the device"""
     probs = [P.diffusion3d(24, seed=1), P.elasticity3d(12, seed=2), P.diffusion3d(13, seed=3)]
