@@ -99,7 +99,8 @@ typedef struct ins_stats {
     int64_t n_active;
     int64_t nnz;
     int64_t device_bytes;   /* device memory held by the context             */
-    double spmv_ms;         /* profiled: total time of the dominant SpMV     */
+    double spmv_ms;         /* profiled: total time of the dominant SpMV
+                               (see ins_set_profiling)                       */
     int64_t spmv_calls;     /* profiled: launches timed                      */
     int64_t sell_values;    /* padded value count of the SELL storage (0 = none) */
     int     sell_patterns;  /* distinct column-offset lists of the SELL storage  */
@@ -133,7 +134,10 @@ int ins_get_stats(const ins_ctx* ctx, ins_stats* out);
 /* Free and total device memory of GPU `device` (hipMemGetInfo), for
  * admission by free HBM.  No reference counterpart. */
 int ins_device_memory(int device, uint64_t* free_bytes, uint64_t* total_bytes);
-/* time every dominant-kernel launch with HIP events (adds small overhead) */
+/* Time every dominant-kernel launch with HIP events (adds small overhead).  A
+ * solve that would run many iterations in one launch (up to some hundred thousand
+ * rows) runs three kernels per iteration instead while profiling is on: the same
+ * iterates, but the times are those kernels' and not the ones of the launch. */
 int ins_set_profiling(ins_ctx* ctx, int on);
 int ins_sync(ins_ctx* ctx);
 

@@ -1499,10 +1499,11 @@ hipError_t ordered(int device, hipStream_t st, F launches)
     if (!o.last) e = hipEventCreateWithFlags(&o.last, hipEventDisableTiming);
     else if (o.stream != st) e = hipStreamWaitEvent(st, o.last, 0);
     if (e != hipSuccess) return e;
-    e = launches();
-    if (e != hipSuccess) return e;
+    // (of several launches the first may run although a later one failed)
+    const hipError_t le = launches();
     o.stream = st;
-    return hipEventRecord(o.last, st);
+    e = hipEventRecord(o.last, st);
+    return le != hipSuccess ? le : e;
 }
 
 template <class K, typename... A>
@@ -1790,6 +1791,9 @@ int sell_cuts(Ctx* c, int bmax, Seg* g)
 {
     Resident& S = c->res;
     const int64_t nsl = c->sell.nslices;
+    // more slices or entries than all segments hold: no cuts, and no search for any
+    const int64_t regs = (int64_t)TASKS * SELL_MAXE;
+    if (nsl > (int64_t)bmax * SELL_MAXR || c->sell.nvals / 64 > bmax * regs) return INS_OK;
     if (S.cut_gen != c->pattern_gen) {
         std::vector<int64_t> ptr((size_t)nsl + 1);
         INS_HIP_CHECK(c, hipMemcpyAsync(ptr.data(), c->sell.slice_ptr.p, ptr.size() * sizeof(int64_t),
@@ -1797,7 +1801,6 @@ int sell_cuts(Ctx* c, int bmax, Seg* g)
         INS_HIP_CHECK(c, hipStreamSynchronize(c->stream));
         const int64_t total = ptr[nsl] / 64;
         // 64 blocks while the registers hold their entries, beyond: all blocks
-        const int64_t regs = (int64_t)TASKS * SELL_MAXE;
         int64_t most = (total + 63) / 64;
         if (most > regs) most = (total + bmax - 1) / bmax;
         std::vector<int32_t> cut;
