@@ -3909,8 +3909,7 @@ struct Server {
     int64_t it = 0;      // batched iterations launched
     int64_t chunks = 0;  // chunks launched
     hipEvent_t ev_sync = nullptr;
-    // the resident launches of a step that has batched kernels too: those
-    // leave most of every compute unit idle, and the chains are independent
+    // the second of two independent chains of a step (server_step)
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     Backoff backoff;     // requests after a launch that gave up
@@ -4028,9 +4027,8 @@ double request_mb(const SlotH& h)
 
 // The resident launches of a step: requests share one while every block has a compute
 // unit (first fit, the largest first: eight requests of 16^3 to 44^3 take three
-// launches, 20.1 ms, and took four in the order of their slots, 21.7).  Beside
-// batched kernels a launch leaves them a quarter of the units (a resident block fills
-// its own): a batch of eight with one that is not resident 23.5 ms, 25.3 without.
+// launches, 20.1 ms, and took four in the order of their slots, 21.7).  Beside the
+// segment kernels they leave a quarter of the units (a resident block fills its own).
 //
 // Launches follow one another, while the batched kernels on segments share three
 // launches among all requests, so many middle-sized requests go faster there, and
@@ -4039,17 +4037,20 @@ double request_mb(const SlotH& h)
 //   70k elastic rows   3: 13.8/14.8/13.6  4: 18.7/16.6/15.4  6: 27.9/19.8/18.8
 //   114k elastic rows  3: 17.0/20.2/18.5  5: 28.8/25.2/26.7   202k: 4: 30.4/36.0/33.7
 //   89k scalar rows    2: 5.6/5.2/6.0     6: 16.8/10.8/12.4   223k: 4: 18.0/15.8/18.8
+// Beside requests on whole vectors, which need the compute units, the others run on
+// the segment kernels (28 requests of 16^3 to 96^3 a second, resident beside them:
+// mean latency 131 ms, 99% 863 ms; on segments 126 and 756).
 // A request that has moved to the segment kernels stays there.  Both have the same
 // bits, so a running request can move between two steps.
 std::vector<std::vector<int>> pack_requests(Server* sv)
 {
-    bool beside = false, segs = false;
+    bool whole = false, segs = false;
     std::vector<int> order;
     for (int s = 0; s < sv->max_slots; s++) {
         const SlotH& h = sv->slots[s];
         if (h.state != INS_SLOT_RUNNING) continue;
         if (h.resident) order.push_back(s);
-        beside |= !h.resident;
+        whole |= !h.seg.g.B;
         segs |= !h.resident && h.seg.g.B > 0;
     }
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
@@ -4061,7 +4062,7 @@ std::vector<std::vector<int>> pack_requests(Server* sv)
     for (int s : order) {
         const SlotH& h = sv->slots[s];
         const int B = h.seg.g.B, all = resident_blocks(h.c->n_cu);
-        const int most = beside ? all * 3 / 4 : all;
+        const int most = segs ? all * 3 / 4 : all;
         size_t g = 0;
         while (g < groups.size() && blocks[g] + B > most) g++;
         if (g == groups.size()) {
@@ -4073,7 +4074,7 @@ std::vector<std::vector<int>> pack_requests(Server* sv)
         blocks[g] += B;
         t_seg += 0.25 * request_mb(h);
     }
-    if (groups.size() > 1 && t_seg < t_res) {
+    if (whole || (groups.size() > 1 && t_seg < t_res)) {
         for (int s : order) sv->slots[s].resident = false;
         groups.clear();
     }
@@ -4299,11 +4300,11 @@ int server_step(Server* sv, int k, int* n_finished)
             if (h.state == INS_SLOT_RUNNING && h.resident &&
                 resident_words(h.c, sv->stream, k, &first[h.cg]) != INS_OK)
                 return sfail(sv, INS_ERR_HIP, h.c->err);
-        // what runs on segments goes beside the kernels on whole vectors, or
-        // resident launches beside the kernels on segments
+        // the kernels on segments go beside those on whole vectors, resident
+        // launches beside the kernels on segments
         const bool resident = !sv->groups.empty(), whole = sv->grid_spmv > 0;
         const bool segs = sv->grid_seg > 0;
-        const bool fork = whole ? resident || segs : resident && segs;
+        const bool fork = segs && (whole || resident);
         hipStream_t st = fork ? sv->side : sv->stream;
         hipStream_t st_seg = whole ? st : sv->stream;
         if (fork) {

@@ -268,18 +268,19 @@ def test_solves_after_a_give_up_keep_their_bits(monkeypatch):
 
 
 # one request of every storage form: scalar slices, node blocks in 3-D and 2-D,
-# full slices (partly prescribed nodes, degree 2), and two too large to be resident
+# full slices (partly prescribed nodes, degree 2), and one too large for segments
 BATCH = [(P.diffusion3d, 17), (P.elasticity3d, 9), (_sheet_2d, 30), (_half_clamped, 8),
          (P.diffusion3d_q2, 7), (_poisson_2d, 50), (P.diffusion3d, 75), (P.elasticity3d, 50)]
 
 
+@pytest.mark.parametrize("batch", [BATCH[:-1], BATCH], ids=["segments", "whole"])
 @pytest.mark.parametrize("polls", [None, "0"], ids=["resident", "given up"])
-def test_batch_of_all_forms_has_the_bits_of_its_solves(polls, monkeypatch):
-    """resident launches beside batched kernels on the second stream; with a
-    bound of no polls the resident requests start again on the batched segment
-    kernels"""
+def test_batch_of_all_forms_has_the_bits_of_its_solves(polls, batch, monkeypatch):
+    """resident launches, or, beside the last request, which is too large for
+    segments, the batched segment kernels on the second stream; with a bound of
+    no polls resident requests start again on those"""
     cs, alone = [], []
-    for make, n in BATCH:
+    for make, n in batch:
         c = abi.Context(0)
         c.load_problem(make(n))
         c.prepare(abi.SOLVE_MIXED, abi.FMT_SELL)
@@ -293,7 +294,7 @@ def test_batch_of_all_forms_has_the_bits_of_its_solves(polls, monkeypatch):
         for _ in range(2):
             slots = [srv.attach(c, 1e-8) for c in cs]
             srv.run_until_done()
-            for (make, n), c, slot, want in zip(BATCH, cs, slots, alone):
+            for (make, n), c, slot, want in zip(batch, cs, slots, alone):
                 state, status, it, rel = srv.poll(slot)
                 assert (state, status) == (abi.SLOT_FINISHED, abi.INS_OK)
                 srv.detach(slot)
